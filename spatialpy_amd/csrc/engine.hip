@@ -183,8 +183,8 @@ struct ssasdpd_engine {
     uint32_t *xx = nullptr;
     double *rrate = nullptr, *srrate = nullptr, *sdrate = nullptr, *Ddiag = nullptr, *qtime = nullptr, *tmin = nullptr;
     double *vol = nullptr;
-    int *targ = nullptr, *ntype = nullptr;
-    int pl = 1, nlev = 0, lev_off[10] = {0}, lev_n[10] = {0}, tree_nodes = 0;
+    int *ntype = nullptr;
+    int pl = 1, tree_nodes = 0;
     size_t lds_bytes = 0;
     QueueState *qs = nullptr;
     int *qwork = nullptr;
@@ -294,7 +294,7 @@ struct ssasdpd_engine {
         if (stage) (void)hipFree(stage);
         pbuf = stage = nullptr;
         pbuf_cap = stage_cap = 0;
-        dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin); dfree(b_targ);
+        dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin);
         dfree(b_qs); dfree(b_seeds);
         dfree(x); dfree(v); dfree(vt); dfree(F); dfree(Fbp); dfree(normal);
         dfree(rho); dfree(old_rho); dfree(Frho); dfree(mass); dfree(nu); dfree(bvf);
@@ -332,7 +332,7 @@ struct ssasdpd_engine {
         dfree(derr_alt);
         dfree(vm_code); dfree(vm_k); dfree(dfn);
         dfree(rx); dfree(jcN); dfree(irN); dfree(prN); dfree(jcG); dfree(irG); dfree(Ndense); dfree(Dmat); dfree(bc);
-        dfree(xx); dfree(rrate); dfree(srrate); dfree(sdrate); dfree(Ddiag); dfree(qtime); dfree(tmin); dfree(targ);
+        dfree(xx); dfree(rrate); dfree(srrate); dfree(sdrate); dfree(Ddiag); dfree(qtime); dfree(tmin);
         dfree(qs); dfree(qwork); dfree(d_psum); dfree(d_words); dfree(d_expo); dfree(d_trace); dfree(derr);
         for (int p = 0; p < NPH; p++)
             for (int k = 0; k < 2; k++) {
@@ -463,27 +463,19 @@ struct ssasdpd_engine {
         if (!pl_valid(p, n))
             throw HipError("too many voxels for the event tree (max 8.3M)", hipErrorUnknown, __FILE__, __LINE__);
         pl = p;
-        lev_n[0] = n;
-        lev_n[1] = (n + 64 * pl - 1) / (64 * pl);
-        lev_off[1] = 0;
-        nlev = 1;
-        tree_nodes = lev_n[1];
-        while (lev_n[nlev] > 1) {
-            lev_n[nlev + 1] = (lev_n[nlev] + TREE_FAN - 1) / TREE_FAN;
-            lev_off[nlev + 1] = tree_nodes;
-            tree_nodes += lev_n[nlev + 1];
-            nlev++;
-        }
-        // the event loop holds level nlev-1 in registers and repairs the
-        // levels below it with at most one level in LDS
-        if (nlev > 3)
-            throw HipError("event tree deeper than three levels", hipErrorUnknown, __FILE__, __LINE__);
-        dfree(tmin); dfree(targ);
+        tree_nodes = (n + 64 * pl - 1) / (64 * pl);
+        dfree(tmin);
         tmin = dalloc<double>(tree_nodes);
-        targ = dalloc<int>(tree_nodes);
-        lds_bytes = ssa_lds_bytes(tree_nodes, S, R, T, nnzN_, nnzG_, n_code, n_consts);
-        if (lds_bytes > 65536)
+        if (admitted_lds(p) > 65536)
             throw HipError("event-loop constants exceed 64 KiB of LDS", hipErrorUnknown, __FILE__, __LINE__);
+        lds_bytes = nsm_lds_bytes(tree_nodes, S, R, T, n_code, n_consts);
+    }
+    // ssa_lds_bytes at node width p, over a tree of the nodes and of the
+    // levels above them, 64 to one
+    size_t admitted_lds(int p) const {
+        int n1 = (n + 64 * p - 1) / (64 * p), nodes = n1;
+        while (n1 > 1) { n1 = (n1 + TREE_FAN - 1) / TREE_FAN; nodes += n1; }
+        return ssa_lds_bytes(nodes, S, R, T, nnzN_, nnzG_, n_code, n_consts);
     }
     // Change the tree width of a built queue: the levels are rebuilt from
     // the firing times, so the event sequence is unchanged.
@@ -637,9 +629,9 @@ struct ssasdpd_engine {
             rrate = dalloc<double>((size_t)n * std::max(R, 1));
             srrate = dalloc<double>(n); sdrate = dalloc<double>(n);
             Ddiag = dalloc<double>((size_t)n * S);
-            qtime = dalloc<double>(n);
-            // event tree: level 1 groups F0 = 64*pl voxels (pl chosen so the
-            // levels above the voxels fit the event loop's LDS), 64 per node above
+            qtime = dalloc<double>((size_t)n + NODE_MAX);
+            // event queue: nodes of 64*pl voxels (pl chosen so that their
+            // bounds fit the event loop's LDS)
             nnzN_ = R > 0 ? d->jcN[R] : 0;
             nnzG_ = d->jcG[S + R];
             int p0 = pl_override ? pl_override : auto_pl(n);
@@ -958,10 +950,8 @@ struct ssasdpd_engine {
         a.Ddiag = Ddiag; a.Dmat = Dmat; a.rx = rx; a.jcN = jcN; a.irN = irN; a.prN = prN; a.jcG = jcG; a.irG = irG;
         a.deg = deg; a.nidx = nidx; a.ntype = ntype; a.Dij = Dij; a.vol = vol;
         a.erow = erow;
-        a.row_w = std::max(1, std::min(W, max_deg_seen));
-        a.qtime = qtime; a.tmin = tmin; a.targ = targ; a.nlev = nlev; a.pl = pl; a.tree_nodes = tree_nodes;
+        a.qtime = qtime; a.tmin = tmin; a.pl = pl; a.tree_nodes = tree_nodes;
         a.lds_bytes = lds_bytes;
-        for (int l = 0; l < 10; l++) { a.lev_off[l] = lev_off[l]; a.lev_n[l] = lev_n[l]; }
         a.qs = qs;
         a.rng_kind = rng_kind; a.seed = seed; a.stream_id = 0; a.words = d_words; a.expo = d_expo; a.n_words = n_words;
         a.textbook = (flags & SSASDPD_FLAG_TEXTBOOK_SELECTION) ? 1 : 0;
@@ -1306,7 +1296,6 @@ struct ssasdpd_engine {
     int bcap = 0;
     uint32_t *b_xx = nullptr;
     double *b_rr = nullptr, *b_sr = nullptr, *b_sd = nullptr, *b_qt = nullptr, *b_tmin = nullptr;
-    int *b_targ = nullptr;
     QueueState *b_qs = nullptr;
     unsigned long long *b_seeds = nullptr;
     std::vector<uint64_t> b_seed_h;
@@ -1314,16 +1303,15 @@ struct ssasdpd_engine {
 
     void batch_alloc(int B) {
         if (B <= bcap) return;
-        dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin); dfree(b_targ);
+        dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin);
         dfree(b_qs); dfree(b_seeds);
         const size_t nn = n;
         b_xx = dalloc<uint32_t>(nn * S * B);
         b_rr = dalloc<double>(nn * std::max(R, 1) * B);
         b_sr = dalloc<double>(nn * B);
         b_sd = dalloc<double>(nn * B);
-        b_qt = dalloc<double>(nn * B);
+        b_qt = dalloc<double>(nn * B + NODE_MAX);
         b_tmin = dalloc<double>((size_t)std::max(tree_nodes, 1) * B);
-        b_targ = dalloc<int>((size_t)std::max(tree_nodes, 1) * B);
         b_qs = dalloc<QueueState>(B);
         b_seeds = dalloc<unsigned long long>(B);
         bcap = B;
@@ -1348,7 +1336,6 @@ struct ssasdpd_engine {
         a.sdrate = b_sd + o * a.bs_n;
         a.qtime = b_qt + o * a.bs_n;
         a.tmin = b_tmin + o * a.bs_tree;
-        a.targ = b_targ + o * a.bs_tree;
         a.qs = b_qs + o;
         if (b < 0) a.seeds = b_seeds;
         else a.seed = b_seed_h[b];
@@ -1490,13 +1477,8 @@ struct ssasdpd_ensemble {
         for (auto *e : eng)
             if (!ssasdpd_engine::pl_valid(p, e->n)) return false;
         for (auto *e : eng)
-            if (ssa_lds_bytes_for(e, p) > 65536) return false;
+            if (e->admitted_lds(p) > 65536) return false;
         return true;
-    }
-    static size_t ssa_lds_bytes_for(const ssasdpd_engine *e, int p) {
-        int n1 = (e->n + 64 * p - 1) / (64 * p), nodes = n1;
-        while (n1 > 1) { n1 = (n1 + TREE_FAN - 1) / TREE_FAN; nodes += n1; }
-        return ssa_lds_bytes(nodes, e->S, e->R, e->T, e->nnzN_, e->nnzG_, e->n_code, e->n_consts);
     }
     void set_pl(int p) {
         for (auto *e : eng) e->set_pl(p);
@@ -1541,7 +1523,7 @@ struct ssasdpd_ensemble {
         HIP_OK(hipEventRecord(e0, st));
         bool any_prog = false;
         for (auto *e : eng) any_prog = any_prog || e->n_code > 0;
-        rdme_take_step_multi(st, d_args, (int)args.size(), pl, max_sr, lds_max(), any_prog);
+        rdme_take_step_multi(st, d_args, (int)args.size(), max_sr, lds_max(), any_prog);
         HIP_OK(hipEventRecord(e1, st));
         HIP_OK(hipStreamSynchronize(st));
         float ms = 0.f;

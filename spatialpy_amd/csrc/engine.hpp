@@ -6,7 +6,7 @@
 //   neighbour lists: ELL, column-major [W][n] for idx (int32), r (FP64 |x_i-x_j|)
 //              and Dij (FP64); deg[n]
 //   RDME: xx uint32 [n][S], rrate FP64 [n][R], srrate/sdrate FP64 [n],
-//         Ddiag FP64 [n][S], firing times FP64 [n] + a 64-ary min tree
+//         Ddiag FP64 [n][S], firing times FP64 [n] and their minima per node
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstddef>
@@ -36,6 +36,7 @@ int report_error(int code, const std::string &msg);
 
 constexpr int WAVE = 64;
 constexpr int TREE_FAN = 64;
+constexpr int NODE_MAX = 2048;   // widest node of the event queue (64 * 32 voxels)
 
 // XCD-aware block order for particle-order kernels: the hardware deals
 // consecutive workgroups round-robin to the 8 XCDs, each with its own L2;
@@ -241,20 +242,13 @@ struct RdmeArgs {
     const int *deg, *nidx, *ntype;
     const double *Dij;
     const EdgeRec *erow;     // the same rows voxel-major (event loop)
-    int row_w;               // no row is longer (<= W)
     double *vol;             // mass/rho per voxel, set by the rates kernel
-    // queue: level 0 = firing times of the voxels; level k >= 1 holds the
-    // (time, voxel) minimum of its children: F0 = 64*pl voxels per level-1
-    // node, 64 nodes per node above.  Levels 1..nlev live in tmin/targ at
-    // lev_off[k]; level nlev is the root.
+    // queue: the voxels' firing times (padded to a whole node) and, per node
+    // of 64*pl voxels, a lower bound of those the event loop has not taken
     double *qtime;
     double *tmin;
-    int *targ;
-    int pl;                  // level-0 children per lane (F0 = 64*pl)
-    int nlev;                // number of levels above level 0 (>= 1)
-    int lev_off[10];
-    int lev_n[10];           // nodes per level (lev_n[0] = n)
-    int tree_nodes;          // sum of lev_n[1..nlev]
+    int pl;
+    int tree_nodes;
     size_t lds_bytes;        // dynamic LDS of the event-loop kernel
     QueueState *qs;
     // random stream
@@ -304,16 +298,15 @@ void rdme_rates(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
 void rdme_queue_build(hipStream_t s, const RdmeArgs &a, void *scan_tmp, int *rank_tmp);
 void rdme_take_step(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
 void tree_rebuild(hipStream_t s, const RdmeArgs &a);
-// one launch over n_models argument blocks (device array), common PL and
-// MS/MR bucket (max over the models of max(S, R)), LDS = max over models
-void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int pl, int max_sr, size_t lds,
-                          bool any_prog);
+// one launch over n_models argument blocks (device array), common MS/MR bucket (max over the models of max(S, R)), LDS = max over models
+void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog);
 void vm_eval_batch(hipStream_t s, const uint32_t *code, int start, const double *K, int x_is_double, int n_x,
                    int n_df, int m, const double *xd, const uint32_t *xu, const double *vol, const double *t,
                    const double *df, double *out);
 // Row permutation of an [n][cols] array of esz-byte elements (4 or 8):
 // gather dst[p] = src[map[p]], or scatter dst[map[p]] = src[p] (sdpd.hip).
 void permute_rows(hipStream_t s, int n, int cols, int esz, const int *map, const void *src, void *dst, bool scatter);
+size_t nsm_lds_bytes(int nodes, int S, int R, int T, int n_code, int n_consts);
 size_t ssa_lds_bytes(int tree_nodes, int S, int R, int T, int nnzN, int nnzG, int n_code = 0, int n_consts = 0);
 
 }  // namespace ssa

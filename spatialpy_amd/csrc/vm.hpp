@@ -185,15 +185,18 @@ __device__ __forceinline__ double vm_apply(int op, int idx, double l, double r) 
 // One evaluation.  XT = uint32_t: species counts read as `int` (a
 // propensity, const int *x); XT = double: concentrations (a deterministic
 // rate, const double *x).  The stack lives in registers (constant indices
-// only).
-template <class XT>
+// only).  Species s is x[s * STRIDE].
+template <class XT, int STRIDE = 1, bool UNIFORM = false>
 __device__ __forceinline__ double vm_run(const uint32_t *code, int pc, const double *K, const XT *x, double vol,
                                          double t, const double *df) {
     double s[VM_STACK];
 #pragma unroll
     for (int k = 0; k < VM_STACK; k++) s[k] = 0.0;
     for (int it = 0; it < VM_MAX_STEPS; it++) {
-        const uint32_t w = code[pc++];
+        // UNIFORM: every active lane runs the same program, so the decoding
+        // and its branches are scalar
+        const uint32_t w = UNIFORM ? (uint32_t)__builtin_amdgcn_readfirstlane((int)code[pc]) : code[pc];
+        pc++;
         const int op = (int)(w & 63u), src = (int)((w >> 6) & 7u), idx = (int)(w >> 10);
         if (op == VM_RET) return s[0];
         if (op == VM_NEG_D) { s[0] = -s[0]; continue; }
@@ -203,8 +206,8 @@ __device__ __forceinline__ double vm_run(const uint32_t *code, int pc, const dou
         switch (src) {
         case VM_S_CONST: b = K[idx]; break;
         case VM_S_X:
-            if constexpr (sizeof(XT) == 4) b = vm_i((int)x[idx]);
-            else b = (double)x[idx];
+            if constexpr (sizeof(XT) == 4) b = vm_i((int)x[idx * STRIDE]);
+            else b = (double)x[idx * STRIDE];
             break;
         case VM_S_VOL: b = vol; break;
         case VM_S_T: b = t; break;
@@ -233,6 +236,12 @@ __device__ __forceinline__ double vm_run(const uint32_t *code, int pc, const dou
 static __device__ __noinline__ double vm_eval_u32(const uint32_t *code, int pc, const double *K, const uint32_t *x,
                                                   double vol, double t, const double *df) {
     return vm_run<uint32_t>(code, pc, K, x, vol, t, df);
+}
+// one program on every active lane, species s of a lane at x[64 s] (the event
+// loop's staged counts)
+static __device__ __noinline__ double vm_eval_wave(const uint32_t *code, int pc, const double *K, const uint32_t *x,
+                                                   double vol, double t, const double *df) {
+    return vm_run<uint32_t, 64, true>(code, pc, K, x, vol, t, df);
 }
 static __device__ __noinline__ double vm_eval_f64(const uint32_t *code, int pc, const double *K, const double *x,
                                                   double vol, double t, const double *df) {
