@@ -950,6 +950,7 @@ struct ssasdpd_engine {
         a.Ddiag = Ddiag; a.Dmat = Dmat; a.rx = rx; a.jcN = jcN; a.irN = irN; a.prN = prN; a.jcG = jcG; a.irG = irG;
         a.deg = deg; a.nidx = nidx; a.ntype = ntype; a.Dij = Dij; a.vol = vol;
         a.erow = erow;
+        a.row_w = std::max(1, std::min(W, max_deg_seen));
         a.qtime = qtime; a.tmin = tmin; a.pl = pl; a.tree_nodes = tree_nodes;
         a.lds_bytes = lds_bytes;
         a.qs = qs;

@@ -232,6 +232,7 @@ void sdpd_pack(hipStream_t s, const SdpdArgs &a);
 // RDME.
 struct RdmeArgs {
     int n, S, R, T, W;
+    int row_w;               // no neighbour row is longer (<= W)
     const double *mass, *rho;
     const int *type;
     uint32_t *xx;

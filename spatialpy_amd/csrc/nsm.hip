@@ -41,10 +41,10 @@
 // nodes brings hundreds of events.
 //
 // Measured (MI355X, time per event, the one-by-one loop with its event tree
-// against the rounds): 40^3 lattice, 200,000 molecules 3.7 -> 0.42 us; 256 of
-// those trajectories at once 14.7 -> 1.8 ns; 2D dam break 3.6 -> 0.47 us; 1M
-// cylinder, 860 events a step, 2.8 -> 0.49 us; 121 voxels 3.5 -> 1.5 us;
-// custom propensities on 144 voxels 30 -> 12.5 us.  A round takes 20,000 to
+// against the rounds): 40^3 lattice, 200,000 molecules 3.7 -> 0.36 us; 256 of
+// those trajectories at once 14.7 -> 1.6 ns; 2D dam break 3.6 -> 0.42 us; 1M
+// cylinder, 860 events a step, 2.8 -> 0.45 us; 121 voxels 3.5 -> 1.5 us;
+// custom propensities on 144 voxels 30 -> 5.2 us.  A round takes 20,000 to
 // 50,000 cycles, most of them latencies (two round trips, LDS, dependent
 // FP64 operations) of a single wavefront.
 #include <hip/hip_runtime.h>
@@ -64,7 +64,7 @@ namespace ssa {
 namespace {
 
 constexpr int FRONT_LOW = 40;      // refill the front below this many entries
-constexpr int FRONT_FILL = 58;     // entries that aims at
+constexpr int FRONT_FILL = 56;     // entries that aims at
 constexpr int NEAR = 512;          // entries of the near list
 constexpr int NEAR_LOW = 32;       // refill the near list below this many
 constexpr int NEAR_FILL = 350;     // entries that aims at, at most
@@ -142,11 +142,11 @@ struct Lds {
     int *qv;               // [NEAR] and voxels
     double *ht;            // [NEAR] times on their way into the front
     int *hv;               // [NEAR] and voxels
-    int *nodes;            // [WAVES][GROUP] nodes to scan
+    int *nodes;            // [WAVES][GROUP] nodes to scan (and 64 places while ranks are checked)
     unsigned *claim;       // [2][CLAIMS] (in the same place as ht, hv)
     Rxn *rx;               // [R]
     double *Dmat;          // [S][T]
-    int *dN;               // [R][S] stoichiometry, dense
+    int *dN;               // [R][MS] stoichiometry, dense
     unsigned *dep;         // [S + R] dependency columns as reaction bitmasks
     unsigned *tot;         // [S] species totals
     struct Scan {          // a scan of the nodes, shared by the wavefronts
@@ -167,7 +167,7 @@ size_t nsm_lds_bytes(int nodes, int S, int R, int T, int n_code, int n_consts) {
     size_t o = a16(sizeof(double) * nodes);
     o += sizeof(double) * 2 * POOL + (sizeof(double) + sizeof(int)) * NEAR + sizeof(int) * WAVES * GROUP;
     o += sizeof(unsigned) * 2 * CLAIMS + sizeof(Lds::Scan);
-    o += a16(sizeof(Rxn) * R) + a16(sizeof(double) * S * T) + a16(sizeof(int) * R * S) + a16(sizeof(unsigned) * (S + R));
+    o += a16(sizeof(Rxn) * R) + a16(sizeof(double) * S * T) + a16(sizeof(int) * R * 16) + a16(sizeof(unsigned) * (S + R));
     o += a16(sizeof(unsigned) * S);
     static_assert(sizeof(Lds::Scan) % 16 == 0, "keeps the next array aligned");
     if (n_code > 0)
@@ -263,7 +263,7 @@ template <int MS, int MR, bool VM> struct Loop {
         }
         double p;
         if (VM && kind == 4) {
-            p = vm_eval_wave(L.vcode, ia, L.vk, L.vmx + lane, vol, t, df);
+            p = vm_run<uint32_t, WAVE, true>(L.vcode, ia, L.vk, L.vmx + lane, vol, t, df);
         } else if (kind == 0) {
             p = k * vol;
         } else {
@@ -285,10 +285,10 @@ template <int MS, int MR, bool VM> struct Loop {
     }
     // The propensities of the reactions in this lane's column `dep` after a
     // change of counts, the changes added in the column's order; lanes' masks
-    // differ, so every reaction of any lane's column is evaluated.
+    // differ, so every reaction of any lane's column is evaluated.  (Models
+    // without custom propensities.)
     __device__ __forceinline__ double update(Voxel<MS, MR> &vx, unsigned dep, double vol, int tp, double t,
                                              const double *df, bool active) const {
-        stage(vx.x);
         double rd = 0.0;
 #pragma unroll
         for (int j = 0; j < MR; j++) {
@@ -551,87 +551,129 @@ template <int MS, int MR, bool VM> struct Loop {
             if (cnt == 0 || before(tau_t, tau_v, far_t, far_v)) { tau_t = far_t; tau_v = far_v; }
             return;
         }
-        double least = INFINITY;
-        for (int k = lane; k < nc; k += WAVE) least = fmin(least, L.qt[k]);
-        least = wave_min(least);
         const int room = WAVE - cnt;
-        double to = fmax(tau_t, least) + gap * (double)(FRONT_FILL - cnt);
-        bool all = !(to < far_t);              // up to the second horizon
-        if (all) to = far_t;
-        // the entries up to `to` move out of the list
-        int g = 0, kept = 0;
-        for (int c = 0; c < nc; c += WAVE) {
-            const int k = c + lane;
-            const double t = k < nc ? L.qt[k] : INFINITY;
-            const int v = k < nc ? L.qv[k] : 0;
-            const bool take = k < nc && (all || t <= to);
-            const unsigned long long h = __ballot(take), s = __ballot(k < nc && !take);
-            sync_wave();
-            if (take) {
-                const int w = g + (int)__popcll(h & below(lane));
-                L.ht[w] = t;
-                L.hv[w] = v;
-            } else if (k < nc) {
-                const int w = kept + (int)__popcll(s & below(lane));
-                L.qt[w] = t;
-                L.qv[w] = v;
+        const double step = gap * (double)(FRONT_FILL - cnt);
+        double from = tau_t, to;
+        bool all;                              // up to the second horizon
+        int g, kept;
+        for (;;) {
+            if (!(from > -INFINITY)) {
+                // the first refill, or nothing within a step of an empty front
+                from = INFINITY;
+                for (int k = lane; k < nc; k += WAVE) from = fmin(from, L.qt[k]);
+                from = wave_min(from);
             }
-            g += (int)__popcll(h);
-            kept += (int)__popcll(s);
+            to = from + step;
+            all = !(to < far_t);
+            // no more of them than one pass can rank (entries of one time
+            // cannot be told apart that way: those take the longer path)
+            for (int it = 0; it < 4; it++) {
+                int m = 0;
+                for (int c = 0; c < nc; c += WAVE)
+                    m += (int)__popcll(__ballot((c + lane < nc) & (all | (L.qt[min(c + lane, NEAR - 1)] <= to))));
+                if (m <= WAVE) break;
+                to = from + (to - from) * (0.9 * WAVE) / (double)m;
+                all = !(to < far_t);
+            }
+            // the entries up to `to` move out of the list
+            g = kept = 0;
+            for (int c = 0; c < nc; c += WAVE) {
+                const int k = c + lane;
+                const bool in = k < nc;
+                const double t = in ? L.qt[k] : INFINITY;
+                const int v = in ? L.qv[k] : 0;
+                const bool take = in & (all | (t <= to));
+                const unsigned long long h = __ballot(take), s = __ballot(in & !take);
+                sync_wave();
+                if (take) {
+                    const int w = g + (int)__popcll(h & below(lane));
+                    L.ht[w] = t;
+                    L.hv[w] = v;
+                } else if (in) {
+                    const int w = kept + (int)__popcll(s & below(lane));
+                    L.qt[w] = t;
+                    L.qv[w] = v;
+                }
+                g += (int)__popcll(h);
+                kept += (int)__popcll(s);
+            }
+            if (g > 0 || cnt > 0) break;
+            from = -INFINITY;
         }
         nc = kept;
         sync_wave();
+        if (g == 0) {
+            tau_t = to;
+            tau_v = INT_MAX;
+            gap *= 2.0;
+            return;
+        }
+        if (!all) gap = 0.5 * (gap + (to - from) / (double)g);
         // their ranks by (time, voxel); the earliest join the front behind its
         // last entry, the others go back
-        int joined = 0;
+        int joined;
         double nt = INFINITY;
         int nvx = INT_MAX;
-        const int cnt0 = cnt;
-        for (int s0 = 0; s0 < g; s0 += WAVE) {
-            const int k = s0 + lane;
-            const double t = k < g ? L.ht[k] : INFINITY;
-            const int v = k < g ? L.hv[k] : INT_MAX;
+        if (g <= WAVE) {
+            const double t = lane < g ? L.ht[lane] : INFINITY;
+            const int v = lane < g ? L.hv[lane] : INT_MAX;
             int rank = 0;
-            for (int i0 = 0; i0 < g; i0 += 8) {
+            for (int i0 = 0; i0 < g; i0 += 4)
 #pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const int i = min(i0 + u, g - 1);
-                    const bool b = before(L.ht[i], L.hv[i], t, v);
-                    rank += b && i0 + u < g ? 1 : 0;
+                for (int u = 0; u < 4; u++) rank += rl_d(t, i0 + u) < t ? 1 : 0;
+            // by time alone two entries of one time share a rank
+            if (lane < g) L.nodes[rank] = lane;
+            sync_wave();
+            if (__ballot(lane < g && L.nodes[rank] != lane)) {
+                rank = 0;
+                for (int i = 0; i < g; i++) rank += before(rl_d(t, i), rl_i(v, i), t, v) ? 1 : 0;
+            }
+            joined = min(g, room);
+            if (lane < g) {
+                if (rank < joined) {
+                    L.ht[rank] = t;
+                    L.hv[rank] = v;
+                } else {
+                    // (the list held it before: there is room)
+                    L.qt[nc + rank - joined] = t;
+                    L.qv[nc + rank - joined] = v;
                 }
             }
-            const bool keep = k < g && rank < room;
-            const unsigned long long back = __ballot(k < g && !keep), h = __ballot(keep);
-            joined += (int)__popcll(h);
-            if (g <= WAVE) {
-                // one pass: the kept entries to their lanes through LDS
-                sync_wave();
-                if (keep) { L.ht[rank] = t; L.hv[rank] = v; }
-                sync_wave();
-                if (lane >= cnt0 && lane < cnt0 + joined) { nt = L.ht[lane - cnt0]; nvx = L.hv[lane - cnt0]; }
-            } else {
-                for (unsigned long long w = h; w; w &= w - 1) {
-                    const int l = (int)__builtin_ctzll(w);
-                    if (lane == cnt0 + rl_i(rank, l)) { nt = rl_d(t, l); nvx = rl_i(v, l); }
-                }
-            }
-            // back into the list (it held them before: there is room)
-            if ((back >> lane) & 1ULL) {
-                const int w = nc + (int)__popcll(back & below(lane));
-                L.qt[w] = t;
-                L.qv[w] = v;
-            }
-            nc += (int)__popcll(back);
-        }
-        if (lane >= cnt0 && lane < cnt0 + joined) { ft = nt; fv = nvx; }
-        cnt = cnt0 + joined;
-        if (joined == g) {
-            if (all) { tau_t = far_t; tau_v = far_v; }
-            else { tau_t = to; tau_v = INT_MAX; }
+            nc += g - joined;
+            sync_wave();
+            if (lane >= cnt && lane < cnt + joined) { nt = L.ht[lane - cnt]; nvx = L.hv[lane - cnt]; }
         } else {
+            joined = room;
+            for (int s0 = 0; s0 < g; s0 += WAVE) {
+                const int k = s0 + lane;
+                const double t = k < g ? L.ht[k] : INFINITY;
+                const int v = k < g ? L.hv[k] : INT_MAX;
+                int rank = 0;
+                for (int i = 0; i < g; i++) rank += before(L.ht[i], L.hv[i], t, v) ? 1 : 0;
+                const unsigned long long back = __ballot(k < g && rank >= room);
+                for (unsigned long long w = __ballot(k < g && rank < room); w; w &= w - 1) {
+                    const int l = (int)__builtin_ctzll(w);
+                    if (lane == cnt + rl_i(rank, l)) { nt = rl_d(t, l); nvx = rl_i(v, l); }
+                }
+                if ((back >> lane) & 1ULL) {
+                    const int w = nc + (int)__popcll(back & below(lane));
+                    L.qt[w] = t;
+                    L.qv[w] = v;
+                }
+                nc += (int)__popcll(back);
+            }
+        }
+        if (lane >= cnt && lane < cnt + joined) { ft = nt; fv = nvx; }
+        cnt += joined;
+        if (joined < g) {
             tau_t = rl_d(ft, cnt - 1);
             tau_v = rl_i(fv, cnt - 1);
-            gap *= fmax(0.25, (double)joined / (double)g);
+        } else if (all) {
+            tau_t = far_t;
+            tau_v = far_v;
+        } else {
+            tau_t = to;
+            tau_v = INT_MAX;
         }
         sync_wave();
     }
@@ -682,7 +724,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
         L.hv = (int *)(L.ht + NEAR);
         L.rx = (Rxn *)take(sizeof(Rxn) * R);
         L.Dmat = (double *)take(sizeof(double) * S * T);
-        L.dN = (int *)take(sizeof(int) * R * S);
+        L.dN = (int *)take(sizeof(int) * R * MS);
         L.dep = (unsigned *)take(sizeof(unsigned) * (S + R));
         L.tot = (unsigned *)take(sizeof(unsigned) * S);
         L.vmx = nullptr;
@@ -696,7 +738,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
         for (int i = tid; i < lp.nn; i += nthr) L.lb[i] = tmin[i];
         for (int i = tid; i < R; i += nthr) L.rx[i] = a.rx[i];
         for (int i = tid; i < S * T; i += nthr) L.Dmat[i] = a.Dmat[i];
-        for (int i = tid; i < R * S; i += nthr) L.dN[i] = 0;
+        for (int i = tid; i < R * MS; i += nthr) L.dN[i] = 0;
         if (tid < S) L.tot[tid] = 0;
         if (tid < S + R) {
             unsigned d = 0;
@@ -705,7 +747,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
         }
         __syncthreads();
         if (tid < R)
-            for (int k = a.jcN[tid]; k < a.jcN[tid + 1]; k++) L.dN[tid * S + a.irN[k]] = a.prN[k];
+            for (int k = a.jcN[tid]; k < a.jcN[tid + 1]; k++) L.dN[tid * MS + a.irN[k]] = a.prN[k];
     }
     // species totals (persistent mode's snapshots)
     if (a.snap_tot) {
@@ -734,7 +776,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
     lp.cnt = lp.nc = 0;
     lp.tau_t = lp.far_t = -INFINITY;
     lp.tau_v = lp.far_v = -1;
-    lp.near_fill = (int)fmin(fmax((double)q.active * 0.03125, 64.0), (double)NEAR_FILL);
+    lp.near_fill = (int)fmin(fmax((double)q.active * 0.25, 64.0), (double)NEAR_FILL);
     if constexpr (Loop<MS, MR, VM>::HELD) {
 #pragma unroll
         for (int j = 0; j < MR; j++) {
@@ -754,7 +796,8 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
     lp.gap = q.nbins > 0 ? (q.U - q.L) / (16.0 * (double)q.nbins) : a.dt;
     if (!(lp.gap > 0.0) || !(lp.gap < INFINITY)) lp.gap = a.dt;
     lp.guess_empty = 1.0;
-    int width = WAVE;     // lanes a round tries: about twice what the last ones kept
+    const int widest = VM ? WAVE / 2 : WAVE;
+    int width = widest;   // lanes a round tries: about twice what the last ones kept
     const bool textbook = a.textbook != 0;
     const double inf = INFINITY;
     int err = 0;
@@ -819,6 +862,11 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
             EdgeRec er[ROW];
 #pragma unroll
             for (int u = 0; u < ROW; u++) er[u] = row[min(u, W - 1)];
+            // and where rows are longer, the next ones
+            EdgeRec en[ROW];
+            if (a.row_w > ROW)
+#pragma unroll
+                for (int u = 0; u < ROW; u++) en[u] = row[min(ROW + u, W - 1)];
             lp.fill_pool(lp.pos + 4ULL * WAVE);
             sync_wave();
 
@@ -829,23 +877,20 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
             for (int q1 = 0; q1 < S + R; q1++) {
                 // outcome q1: species q1 leaves, or reaction q1 - S fires
                 const int r = q1 - S;
+                const bool can = on && (r < 0 ? pick(vx.x, q1) > 0 : pick(vx.r, r) > 0.0);
+                if (!__ballot(can)) continue;
                 Voxel<MS, MR> w = vx;
                 double sdn = vx.sd;
-                bool can = false;
 #pragma unroll
                 for (int s = 0; s < MS; s++) {
-                    const int d = s < S ? (r < 0 ? (s == q1 ? -1 : 0) : L.dN[r * S + s]) : 0;
-                    if (d != 0) {
-                        if (s == q1) can = vx.x[s] > 0;
-                        w.x[s] += (uint32_t)d;
-                        sdn += Dd[s] * d;
-                    }
+                    const int d = r < 0 ? (s == q1 ? -1 : 0) : L.dN[r * MS + s];
+                    w.x[s] += (uint32_t)d;
+                    sdn += Dd[s] * d;
                 }
-                if (r >= 0) can = pick(vx.r, r) > 0.0;
-                const bool amb = on && can && !(sdn > 1e-9 * vx.sd);
+                const bool amb = can && !(sdn > 1e-9 * vx.sd);
                 if (!__ballot(amb)) continue;
                 bool empty;
-                if (VM) {
+                if constexpr (VM) {
                     empty = lp.guess_empty != 0.0;
                 } else {
                     const double srn = vx.sr + lp.update(w, L.dep[q1], vol, tsv, t, df, amb);
@@ -865,7 +910,15 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
 #pragma unroll
             for (int s = 0; s < MS; s++)
                 cs[s] = s == 0 ? Dd[0] * vx.x[0] : cs[s > 0 ? s - 1 : 0] + Dd[s] * vx.x[s];
-            int c = on ? (share > 0.5 ? 2 : (emS ? 3 : 4)) : 0, ex = 0, which = 0;
+            // most lanes draw a number that hangs on reaction or hop alone
+            unsigned canS = 0, canR = 0;
+#pragma unroll
+            for (int s = 0; s < MS; s++) canS |= vx.x[s] > 0 && Dd[s] > 0.0 ? 1u << s : 0u;
+#pragma unroll
+            for (int j = 0; j < MR; j++) canR |= vx.r[j] > 0.0 ? 1u << j : 0u;
+            const bool plain = !__ballot(on && ((emS && (canS & ~emS)) || (emR && (canR & ~emR))));
+            const int cR = emR ? 1 : 2, cS = emS ? 3 : 4;
+            int c = on ? (share > 0.5 ? cR : cS) : 0, ex = 0, which = 0;
             bool react = false, over = false, act = false, hop = false;
             bool noop = false;       // the event changes nothing and leaves the queue as it is
             int forced = -1;         // lane 0's choice, when the first selection ran past the last entry
@@ -874,28 +927,36 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
             double rand1 = 0.0;
             unsigned long long p0 = 0, cut = 0;
             for (int redo = 0;; redo++) {
-                for (int it = 0; it <= WAVE; it++) {
-                    ex = scan_add(c) - c;
-                    rand1 = lp.uni(lp.pos + ex);
-                    react = rand1 <= share;
+                // the first entry whose running sum the value does not pass
+                auto choose = [&]() {
                     const double rv = react ? (textbook ? rand1 * totrate : rand1 * vx.sr)
                                             : (textbook ? rand1 * totrate - vx.sr : rand1 * vx.sd);
-                    // the first entry whose running sum the value does not pass
                     int wr = R, ws = S;
 #pragma unroll
                     for (int j = MR - 1; j >= 0; j--) wr = ((j < R) & !(rv > cr[j])) ? j : wr;
 #pragma unroll
                     for (int s = MS - 1; s >= 0; s--) ws = ((s < S) & !(rv > cs[s])) ? s : ws;
                     which = react ? wr : ws;
-                    const int gone = (int)(((react ? emR : emS) >> which) & 1u);
-                    const int cn = react ? 2 - gone : (selfx == ex ? 4 : 4 - gone);
-                    const bool ch = on && cn != c;
-                    if (!__ballot(ch)) break;
-                    if (on) c = cn;
+                };
+                for (int it = 0; it <= WAVE; it++) {
+                    ex = scan_add(c) - c;
+                    rand1 = lp.uni(lp.pos + ex);
+                    react = rand1 <= share;
+                    int cn = react ? cR : cS;
+                    if (!plain) {
+                        choose();
+                        const int gone = (int)(((react ? emR : emS) >> which) & 1u);
+                        cn = react ? 2 - gone : 4 - gone;
+                    }
+                    if (!react && selfx == ex) cn = 4;
+                    cn = on ? cn : 0;
+                    if (!__ballot(cn != c)) break;
+                    c = cn;
                 }
+                choose();
                 p0 = lp.pos + (unsigned long long)ex;
 
-                // lane 0's selections that ran past the last entry
+                // ---- lane 0's selections that ran past the last entry
                 // (simulate_rdme.cpp:262-294, 322-349); other lanes wait for
                 // their turn as lane 0.  cum: what the selection's sum ended at
                 over = on && (react ? which >= R : which >= S);
@@ -966,7 +1027,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 hop = act && !react;
                 spec = hop ? which : 0;
 
-                // the hop's destination: the neighbour row in list order
+                // ---- the hop's destination: the neighbour row in list order
                 const double r2 = lp.uni(p0 + 1);
                 double rand2 = r2 * pick(Dd, spec);
                 jd = -1;
@@ -978,9 +1039,17 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                         double cum2 = 0.0;
                         for (int k0 = 0; k0 < dg && jd < 0; k0 += ROW) {
                             if (held != k0) {
+                                if (held == k0 - ROW) {
 #pragma unroll
-                                for (int u = 0; u < ROW; u++) er[u] = row[min(k0 + u, dg - 1)];
+                                    for (int u = 0; u < ROW; u++) er[u] = en[u];
+                                } else {
+#pragma unroll
+                                    for (int u = 0; u < ROW; u++) er[u] = row[min(k0 + u, dg - 1)];
+                                }
                                 held = k0;
+                                if (k0 + ROW < dg)
+#pragma unroll
+                                    for (int u = 0; u < ROW; u++) en[u] = row[min(k0 + ROW + u, dg - 1)];
                             }
 #pragma unroll
                             for (int u = 0; u < ROW; u++) {
@@ -1044,7 +1113,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
 #pragma unroll
                 for (int s = 0; s < MS; s++)
                     if (s < S) {
-                        const int d = L.dN[which * S + s];
+                        const int d = L.dN[which * MS + s];
                         if (d != 0) {
                             vx.x[s] += (uint32_t)d;
                             vx.sd += Dd[s] * d;
@@ -1055,13 +1124,51 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 for (int s = 0; s < MS; s++)
                     if (s == spec) { vx.x[s] -= 1u; vd.x[s] += 1u; }
             }
-            if (R > 0) {
+            const bool there = mv && !self;
+            if constexpr (VM) {
+                // an evaluation costs 7,000 cycles whatever the lanes hold: the
+                // upper half-wave takes the lower one's destinations (the
+                // 144-voxel model 97 -> 62 ms)
+                const int peer = lane & 31;
+                const bool up = lane >= 32;
+                uint32_t xc[MS];
+#pragma unroll
+                for (int s = 0; s < MS; s++) {
+                    const uint32_t o = (uint32_t)__shfl((int)vd.x[s], peer, WAVE);
+                    xc[s] = up ? o : vx.x[s];
+                }
+                const double vol_c = __shfl(vol, peer, WAVE), t_c = __shfl(t, peer, WAVE);
+                const int tds_c = __shfl(tds, peer, WAVE), dv_c = __shfl(dv, peer, WAVE);
+                const unsigned dep_c = (unsigned)__shfl((int)(up ? 0u : dep), peer, WAVE);
+                const bool on_c = up ? __shfl(there ? 1 : 0, peer, WAVE) != 0 : act;
+                const int at_c = up ? dv_c : sv, tp_c = up ? tds_c : tsv;
+                const double *const df_c = a.data_fn ? a.data_fn + (size_t)at_c * a.n_df : nullptr;
+                lp.stage(xc);
+                double rd = 0.0, rdd = 0.0;
+                for (int j = 0; j < R; j++) {
+                    const bool now = on_c && ((dep_c >> j) & 1u);
+                    if (!__ballot(now)) continue;
+                    const double p = lp.template prop<true>(j, xc, vol_c, tp_c, t_c, df_c);
+                    const double pd = __shfl(p, (lane & 31) + 32, WAVE);
+                    const bool mine = ((dep >> j) & 1u) && act && !up;
+#pragma unroll
+                    for (int u = 0; u < MR; u++)
+                        if (u == j && mine) {
+                            rd += p - vx.r[u];
+                            vx.r[u] = p;
+                            if (there) {
+                                rdd += pd - vd.r[u];
+                                vd.r[u] = pd;
+                            }
+                        }
+                }
+                if (act) vx.sr += rd;
+                if (there) vd.sr += rdd;
+            } else if (R > 0) {
                 const double rd = lp.update(vx, dep, vol, tsv, t, df, act);
                 if (act) vx.sr += rd;
-                const bool there = mv && !self;
                 if (__ballot(there)) {
-                    const double *const dfd = a.data_fn ? a.data_fn + (size_t)dv * a.n_df : nullptr;
-                    const double rdd = lp.update(vd, dep, vol, tds, t, dfd, there);
+                    const double rdd = lp.update(vd, dep, vol, tds, t, nullptr, there);
                     if (there) vd.sr += rdd;
                 }
             }
@@ -1139,7 +1246,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 if (o < WAVE) lp.guess_empty = rl_i(used, o) < rl_i(c, o) ? 1.0 : 0.0;
             }
             const bool done = act && lane < P;
-            width = P == K ? min(2 * width, WAVE) : max(8, min(WAVE, (width + 3 * P + 8) / 2));
+            width = P == K ? min(2 * width, widest) : max(8, min(widest, (width + 3 * P + 8) / 2));
 
             // ---- store
             const unsigned long long m_done = __ballot(done), m_hop = __ballot(done && mv);
@@ -1168,7 +1275,7 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 }
                 if (a.snap_tot && react)
                     for (int s = 0; s < S; s++) {
-                        const int d = L.dN[which * S + s];
+                        const int d = L.dN[which * MS + s];
                         if (d != 0) atomicAdd(L.tot + s, (unsigned)d);
                     }
                 if (a.trace) {

@@ -80,15 +80,15 @@ __device__ __forceinline__ double vm_i(int v) { return (double)v; }
 // reference's x86-64 build)
 __device__ __forceinline__ int vm_wrap(long long v) { return (int)(unsigned)(unsigned long long)v; }
 
-__device__ __forceinline__ double vm_call1(int f, double a) {
+// The interpreter is inlined where it is used, with the functions that take
+// a few registers; the others are a call (a call that may use them all saves
+// and restores some 250 registers per evaluation, 10,000 cycles a wavefront).
+static __device__ __noinline__ double vm_heavy1(int f, double a) {
     switch (f) {
-    case 0: return exp(a);
-    case 1: return log(a);
     case 2: return log10(a);
     case 3: return log2(a);
     case 4: return log1p(a);
     case 5: return expm1(a);
-    case 6: return sqrt(a);
     case 7: return sin(a);
     case 8: return cos(a);
     case 9: return tan(a);
@@ -104,10 +104,28 @@ __device__ __forceinline__ double vm_call1(int f, double a) {
     case 19: return erf(a);
     case 20: return erfc(a);
     case 21: return lgamma(a);
+    default: return __builtin_nan("");
+    }
+}
+__device__ __forceinline__ double vm_call1(int f, double a) {
+    switch (f) {
+    case 0: return exp(a);
+    case 1: return log(a);
+    case 6: return sqrt(a);
     case 22: return fabs(a);
     case 23: return floor(a);
     case 24: return ceil(a);
-    default: return trunc(a);
+    case 25: return trunc(a);
+    default: return vm_heavy1(f, a);
+    }
+}
+static __device__ __noinline__ double vm_heavy2(int f, double a, double b) {
+    switch (f) {
+    case 0: return pow(a, b);
+    case 1: return atan2(a, b);
+    case 2: return hypot(a, b);
+    case 3: return fmod(a, b);
+    default: return remainder(a, b);
     }
 }
 // x^n for integral |n| <= 64 rounded once from a double-double product
@@ -141,16 +159,13 @@ __device__ __forceinline__ double vm_pow(double x, double y) {
         if (isfinite(r) && fabs(r) >= 0x1p-1000 && fabs(r) <= 0x1p1000) return r;
     }
     if (y == 0.5 && x > 0.0 && isfinite(x)) return sqrt(x);
-    return pow(x, y);
+    return vm_heavy2(0, x, y);
 }
 __device__ __forceinline__ double vm_call2(int f, double a, double b) {
     switch (f - VM_FUNC2_BASE) {
     case 0: return vm_pow(a, b);
-    case 1: return atan2(a, b);
-    case 2: return hypot(a, b);
-    case 3: return fmod(a, b);
     case 4: return copysign(a, b);
-    default: return remainder(a, b);
+    default: return vm_heavy2(f - VM_FUNC2_BASE, a, b);
     }
 }
 
@@ -236,12 +251,6 @@ __device__ __forceinline__ double vm_run(const uint32_t *code, int pc, const dou
 static __device__ __noinline__ double vm_eval_u32(const uint32_t *code, int pc, const double *K, const uint32_t *x,
                                                   double vol, double t, const double *df) {
     return vm_run<uint32_t>(code, pc, K, x, vol, t, df);
-}
-// one program on every active lane, species s of a lane at x[64 s] (the event
-// loop's staged counts)
-static __device__ __noinline__ double vm_eval_wave(const uint32_t *code, int pc, const double *K, const uint32_t *x,
-                                                   double vol, double t, const double *df) {
-    return vm_run<uint32_t, 64, true>(code, pc, K, x, vol, t, df);
 }
 static __device__ __noinline__ double vm_eval_f64(const uint32_t *code, int pc, const double *K, const double *x,
                                                   double vol, double t, const double *df) {
