@@ -169,7 +169,6 @@ struct ssasdpd_engine {
     void *kd_work = nullptr;
     size_t kd_work_sz = 0;
     void *scan_tmp = nullptr;
-    void *scan_tmp_q = nullptr;   // the queue build's (it can run beside a binning)
     // chemistry constants
     Rxn *rx = nullptr;
     // expression-VM programs of kind-4 reactions, data functions [n][n_df]
@@ -187,8 +186,7 @@ struct ssasdpd_engine {
     int pl = 1, tree_nodes = 0;
     size_t lds_bytes = 0;
     QueueState *qs = nullptr;
-    int *qwork = nullptr;
-    double *d_psum = nullptr;
+    char *qwork = nullptr;
     // random stream
     int rng_kind = 0;
     uint64_t seed = 0;
@@ -295,7 +293,7 @@ struct ssasdpd_engine {
         pbuf = stage = nullptr;
         pbuf_cap = stage_cap = 0;
         dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin);
-        dfree(b_qs); dfree(b_seeds);
+        dfree(b_qs); dfree(b_seeds); dfree(b_qwork);
         dfree(x); dfree(v); dfree(vt); dfree(F); dfree(Fbp); dfree(normal);
         dfree(rho); dfree(old_rho); dfree(Frho); dfree(mass); dfree(nu); dfree(bvf);
         dfree(type); dfree(solid); dfree(C); dfree(Q);
@@ -327,13 +325,11 @@ struct ssasdpd_engine {
         kd_work = nullptr;
         if (scan_tmp) (void)hipFree(scan_tmp);
         scan_tmp = nullptr;
-        if (scan_tmp_q) (void)hipFree(scan_tmp_q);
-        scan_tmp_q = nullptr;
         dfree(derr_alt);
         dfree(vm_code); dfree(vm_k); dfree(dfn);
         dfree(rx); dfree(jcN); dfree(irN); dfree(prN); dfree(jcG); dfree(irG); dfree(Ndense); dfree(Dmat); dfree(bc);
         dfree(xx); dfree(rrate); dfree(srrate); dfree(sdrate); dfree(Ddiag); dfree(qtime); dfree(tmin);
-        dfree(qs); dfree(qwork); dfree(d_psum); dfree(d_words); dfree(d_expo); dfree(d_trace); dfree(derr);
+        dfree(qs); dfree(qwork); dfree(d_words); dfree(d_expo); dfree(d_trace); dfree(derr);
         for (int p = 0; p < NPH; p++)
             for (int k = 0; k < 2; k++) {
                 if (ev_a[p][k]) (void)hipEventDestroy(ev_a[p][k]);
@@ -534,7 +530,6 @@ struct ssasdpd_engine {
         }
         derr = dalloc<DevErr>(1);
         if (ps) derr_alt = dalloc<DevErr>(1);
-        d_psum = dalloc<double>(2);
         kd.parent = dalloc<int>(2 * (size_t)n + 2); kd.depth = dalloc<int>(2 * (size_t)n + 2);
         kd.cd = dalloc<int>(2 * (size_t)n + 2); kd.cv = dalloc<double>(2 * (size_t)n + 2);
         kd.is_hi = dalloc<int>(2 * (size_t)n + 2); kd.leaf_of = dalloc<int>(n);
@@ -542,7 +537,6 @@ struct ssasdpd_engine {
         HIP_OK(hipMalloc(&kd_work, kd_work_sz));
         size_t scan_sz = std::max(scan_tmp_bytes(4LL * n + (1 << 20) + 8), scan_tmp_bytes(n + 8));
         HIP_OK(hipMalloc(&scan_tmp, scan_sz));
-        HIP_OK(hipMalloc(&scan_tmp_q, scan_tmp_bytes(n + 8)));
         alloc_lists(dim == 3 ? 40 : (dim == 2 ? 16 : 4));
 
         // constants
@@ -642,8 +636,7 @@ struct ssasdpd_engine {
             layout_tree(p0);
             vol = dalloc<double>(n);
             qs = dalloc<QueueState>(1);
-            qwork = (int *)dalloc<char>(sizeof(double) * (size_t)n + sizeof(int) * 4 * ((size_t)n + 1) + 64 +
-                                        sizeof(double) * 512);
+qwork = dalloc<char>(q_work_bytes(n));
         }
         if (Sc > 0 && Rc > 0 && d->N_dense) {
             Ndense = dalloc<int>((size_t)Sc * Rc);
@@ -963,7 +956,7 @@ struct ssasdpd_engine {
         a.dt = dt;
         a.endTime = static_domain ? nt * dt : a.t0 + dt;
         a.step = step;
-        a.psum_out = d_psum;
+        a.qwork = qwork;
         a.vm_code = vm_code; a.vm_k = vm_k; a.vm_ncode = n_code; a.vm_nk = n_consts;
         a.data_fn = dfn; a.n_df = n_df;
         return a;
@@ -1185,8 +1178,7 @@ struct ssasdpd_engine {
     bool prepare_static() {
         particle_phase(0);
         RdmeArgs ra = rdme_args(0);
-        rdme_rates(st, ra);
-        rdme_queue_build(st, ra, scan_tmp_q, qwork);
+        rdme_queue_build(st, ra);
         QueueState q;
         d2h(st, &q, qs, 1);
         HIP_OK(hipStreamSynchronize(st));
@@ -1229,8 +1221,7 @@ struct ssasdpd_engine {
             bool qpend = false;
             if (build) {
                 ph_begin(3);
-                rdme_rates(st, ra);
-                rdme_queue_build(st, ra, scan_tmp_q, qwork);
+                rdme_queue_build(st, ra);
                 ph_end(3);
                 if (static_domain) {
                     // whether the queue holds an event (a static domain then
@@ -1299,13 +1290,13 @@ struct ssasdpd_engine {
     double *b_rr = nullptr, *b_sr = nullptr, *b_sd = nullptr, *b_qt = nullptr, *b_tmin = nullptr;
     QueueState *b_qs = nullptr;
     unsigned long long *b_seeds = nullptr;
-    std::vector<uint64_t> b_seed_h;
+    char *b_qwork = nullptr;
     std::vector<char> b_init;
 
     void batch_alloc(int B) {
         if (B <= bcap) return;
         dfree(b_xx); dfree(b_rr); dfree(b_sr); dfree(b_sd); dfree(b_qt); dfree(b_tmin);
-        dfree(b_qs); dfree(b_seeds);
+        dfree(b_qs); dfree(b_seeds); dfree(b_qwork);
         const size_t nn = n;
         b_xx = dalloc<uint32_t>(nn * S * B);
         b_rr = dalloc<double>(nn * std::max(R, 1) * B);
@@ -1315,12 +1306,12 @@ struct ssasdpd_engine {
         b_tmin = dalloc<double>((size_t)std::max(tree_nodes, 1) * B);
         b_qs = dalloc<QueueState>(B);
         b_seeds = dalloc<unsigned long long>(B);
+        b_qwork = dalloc<char>(q_work_bytes(n) * B);
         bcap = B;
     }
 
-    // The arguments of trajectory b alone (queue build), or of the whole
-    // batch (b < 0: base pointers plus strides for the event loop).
-    RdmeArgs batch_args(unsigned step, int b) {
+    // The arguments of the whole batch: base pointers plus strides.
+    RdmeArgs batch_args(unsigned step) {
         RdmeArgs a = rdme_args(step);
         const size_t nn = n;
         a.bs_xx = nn * S;
@@ -1330,16 +1321,16 @@ struct ssasdpd_engine {
         a.rng_kind = 0;
         a.words = nullptr; a.expo = nullptr; a.n_words = 0;
         a.trace = nullptr; a.trace_cap = 0;
-        const size_t o = b < 0 ? 0 : (size_t)b;
-        a.xx = b_xx + o * a.bs_xx;
-        a.rrate = b_rr + o * a.bs_rr;
-        a.srrate = b_sr + o * a.bs_n;
-        a.sdrate = b_sd + o * a.bs_n;
-        a.qtime = b_qt + o * a.bs_n;
-        a.tmin = b_tmin + o * a.bs_tree;
-        a.qs = b_qs + o;
-        if (b < 0) a.seeds = b_seeds;
-        else a.seed = b_seed_h[b];
+        a.xx = b_xx;
+        a.rrate = b_rr;
+        a.srrate = b_sr;
+        a.sdrate = b_sd;
+        a.qtime = b_qt;
+        a.tmin = b_tmin;
+        a.qs = b_qs;
+        a.seeds = b_seeds;
+        a.qwork = b_qwork;
+        a.bs_qwork = q_work_bytes(n);
         return a;
     }
 
@@ -1349,7 +1340,6 @@ struct ssasdpd_engine {
         r.seed = seeds[0];
         reset(&r);
         batch_alloc(B);
-        b_seed_h.assign(seeds, seeds + B);
         b_init.assign(B, 0);
         h2d(st, b_seeds, (const unsigned long long *)seeds, B);
         const size_t nn = n;
@@ -1369,14 +1359,14 @@ struct ssasdpd_engine {
         int rc = check(step);
         if (rc) return rc;
         if (S > 0 && !(flags & SSASDPD_FLAG_NO_RDME)) {
-            bool any = false;
+            // a static domain's queues are built once; those that held no event
+            // are tried again
+            const bool any = !static_domain || !batch_all_init();
             ph_begin(3);
-            for (int b = 0; b < B; b++) {
-                if (static_domain && b_init[b]) continue;
-                RdmeArgs ra = batch_args(step, b);
-                rdme_rates(st, ra);
-                rdme_queue_build(st, ra, scan_tmp_q, qwork);
-                any = true;
+            if (any) {
+                RdmeArgs ra = batch_args(step);
+                ra.only_new = static_domain ? 1 : 0;
+                rdme_queue_build(st, ra, B);
             }
             ph_end(3);
             std::vector<QueueState> q(B);
@@ -1386,7 +1376,7 @@ struct ssasdpd_engine {
                 for (int b = 0; b < B; b++) if (q[b].initialized == 1) b_init[b] = 1;
             }
             ph_begin(4);
-            rdme_take_step(st, batch_args(step, -1), B);
+            rdme_take_step(st, batch_args(step), B);
             ph_end(4);
             rc = batch_check(B, step);
         }
@@ -1850,7 +1840,7 @@ int ssasdpd_run_batch(ssasdpd_engine *e, int32_t n_traj, const uint64_t *seeds, 
             const uint32_t seg = std::min<uint32_t>({e->nt, std::max<uint32_t>(next, step + 1), step + FUSED_SEGMENT});
             int rc = e->particle_steps(step, seg, {}, [](size_t) {});
             if (rc) return rc;
-            e->ssa_fused(e->batch_args(step, -1), B, seg, {}, nullptr, 0, nullptr);
+            e->ssa_fused(e->batch_args(step), B, seg, {}, nullptr, 0, nullptr);
             rc = e->batch_check(B, seg - 1);
             if (rc) return rc;
             step = seg - 1;
@@ -1863,7 +1853,7 @@ int ssasdpd_run_batch(ssasdpd_engine *e, int32_t n_traj, const uint64_t *seeds, 
             int rc = e->particle_steps(step, e->nt, sst, [&](size_t j) { snap_shared(ks[j], sst[j]); });
             if (rc) return rc;
             uint32_t *d_xx = (counts && e->S > 0) ? dalloc<uint32_t>(per * K * B) : nullptr;
-            e->ssa_fused(e->batch_args(step, -1), B, e->nt, sst, d_xx, per * K, nullptr);
+            e->ssa_fused(e->batch_args(step), B, e->nt, sst, d_xx, per * K, nullptr);
             rc = e->batch_check(B, e->nt - 1);
             for (int j = 0; j < K && !rc; j++) {
                 if (d_xx)

@@ -266,8 +266,11 @@ struct RdmeArgs {
     unsigned long long max_events;
     double t0, dt, endTime;
     unsigned step;
-    double *psum_out;
-    int *active_out;
+    // the queue build's work space (q_work_bytes per trajectory); only_new:
+    // trajectories whose queue runs are left alone
+    char *qwork;
+    size_t bs_qwork;
+    int only_new;
     // batched ensembles: trajectory b = blockIdx.x (rates: blockIdx.y) uses
     // its own counts / rates / queue at these element strides; neighbour
     // lists, Ddiag and vol are shared
@@ -295,10 +298,11 @@ struct RdmeArgs {
 // Ddiag from this step's lists, for models with more than FIN_MAX_SPECIES
 // species (the search's finish forms it otherwise; k_bvf forms vol)
 void rdme_diag(hipStream_t s, const RdmeArgs &a);
-void rdme_rates(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
-void rdme_queue_build(hipStream_t s, const RdmeArgs &a, void *scan_tmp, int *rank_tmp);
+// rates, then the event queue built from them
+void rdme_queue_build(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
+size_t q_work_bytes(int n);
 void rdme_take_step(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
-void tree_rebuild(hipStream_t s, const RdmeArgs &a);
+void tree_rebuild(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
 // one launch over n_models argument blocks (device array), common MS/MR bucket (max over the models of max(S, R)), LDS = max over models
 void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog);
 void vm_eval_batch(hipStream_t s, const uint32_t *code, int start, const double *K, int x_is_double, int n_x,
