@@ -304,11 +304,22 @@ struct KdWork {
     unsigned long long *s_min, *s_max;          // [3][cap]
     int *n_start, *n_n, *n_node;                // next level
     double *n_lo, *n_hi;                        // [3][cap]
-    int *counters;                              // [0] next segs, [1] nodes
+    // (cells that one workgroup finishes are kept at the far end of the n_
+    // arrays, from cap - 1 down: a level has at most n / 1025 others)
+    int *counters;                              // [0] next segs, [1] nodes, [2] cells kept for k_kd_local, [3] a cell had no split
     void *scan_tmp;
 };
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Cells of up to this many points are split down to single points by one
+// workgroup (k_kd_local), a point per thread.  A level over the whole array is
+// 27 launches and a wait for the host, about 100 us however small its cells
+// are, and a tree has some log2(n) + 4 levels: with the last ten of them in one
+// launch the tree of 64,000 points takes 0.6 instead of 1.9 ms, of 121 points
+// 0.04 instead of 0.7 ms.  1,024: the most a workgroup holds with a point per
+// thread, at 85 KB of LDS.
+constexpr int KD_LOCAL = 1024;
 
 size_t kd_work_bytes(int n) {
     size_t cap = (size_t)n + 1;
@@ -382,6 +393,17 @@ __global__ void k_kd_root(const double *bb, int n, int dim, KdWork w, KdDev kd, 
     kd.cv[0] = 0.0;
     w.counters[1] = 1;
     if (n == 1) kd.leaf_of[0] = 0;
+    // a tree of one workgroup's points: the root is the one cell kept for it
+    // (the box was read above: with n = 1 the arrays' ends are their starts)
+    if (n > 1 && n <= KD_LOCAL) {
+        w.n_start[cap - 1] = 0;
+        w.n_n[cap - 1] = n;
+        w.n_node[cap - 1] = 0;
+        for (int d = 0; d < 3; d++) {
+            w.n_lo[(size_t)d * cap + cap - 1] = w.s_lo[(size_t)d * cap];
+            w.n_hi[(size_t)d * cap + cap - 1] = w.s_hi[(size_t)d * cap];
+        }
+    }
 }
 
 __global__ void k_kd_mm_init(int nseg, unsigned long long *mn, unsigned long long *mx, int cap) {
@@ -414,34 +436,58 @@ __global__ void k_kd_minmax(const double *pts, int n, int dim, const int *perm, 
     }
 }
 
-// sl_midpt_split's choice of cut dimension and value (kd_split.cpp:146-188).
-__global__ void k_kd_choose(int nseg, int dim, KdWork w, int cap) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
+// sl_midpt_split's choice of cut dimension and value (kd_split.cpp:146-188)
+// for the box lo, hi and the points' extent mn, mx; mode 1 (2): the cut slid
+// to the least (largest) coordinate.
+__device__ __forceinline__ void kd_choose(const double lo[3], const double hi[3], const double mn[3],
+                                          const double mx[3], int dim, int &cut_dim, double &cv, int &mode) {
     const double ERR = 0.001;
-    double lo[3], hi[3];
-    for (int d = 0; d < 3; d++) { lo[d] = w.s_lo[(size_t)d * cap + s]; hi[d] = w.s_hi[(size_t)d * cap + s]; }
     double max_length = hi[0] - lo[0];
     for (int d = 1; d < dim; d++) {
         double length = hi[d] - lo[d];
         if (length > max_length) max_length = length;
     }
-    double max_spread = -1;
-    int cut_dim = 0;
-    for (int d = 0; d < dim; d++) {
-        if ((hi[d] - lo[d]) >= (1 - ERR) * max_length) {
-            double spr = dkey_inv(w.s_max[(size_t)d * cap + s]) - dkey_inv(w.s_min[(size_t)d * cap + s]);
-            if (spr > max_spread) { max_spread = spr; cut_dim = d; }
+    double max_spread = -1, c_lo = lo[0], c_hi = hi[0], c_mn = mn[0], c_mx = mx[0];
+    cut_dim = 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        if (d < dim && (hi[d] - lo[d]) >= (1 - ERR) * max_length) {
+            double spr = mx[d] - mn[d];
+            if (spr > max_spread) {
+                max_spread = spr;
+                cut_dim = d;
+                c_lo = lo[d]; c_hi = hi[d]; c_mn = mn[d]; c_mx = mx[d];
+            }
         }
     }
-    double ideal = (lo[cut_dim] + hi[cut_dim]) / 2;
-    double mn = dkey_inv(w.s_min[(size_t)cut_dim * cap + s]);
-    double mx = dkey_inv(w.s_max[(size_t)cut_dim * cap + s]);
-    double cv;
-    int mode = 0;
-    if (ideal < mn) { cv = mn; mode = 1; }
-    else if (ideal > mx) { cv = mx; mode = 2; }
+    const double ideal = (c_lo + c_hi) / 2;
+    mode = 0;
+    if (ideal < c_mn) { cv = c_mn; mode = 1; }
+    else if (ideal > c_mx) { cv = c_mx; mode = 2; }
     else cv = ideal;
+}
+// n_lo rule (kd_split.cpp:208-212)
+__device__ __forceinline__ int kd_n_lo(int mode, int cnt, int br1, int br2) {
+    if (mode == 1) return 1;
+    if (mode == 2) return cnt - 1;
+    if (br1 > cnt / 2) return br1;
+    if (br2 < cnt / 2) return br2;
+    return cnt / 2;
+}
+
+__global__ void k_kd_choose(int nseg, int dim, KdWork w, int cap) {
+    int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nseg) return;
+    double lo[3], hi[3], mn[3], mx[3];
+    for (int d = 0; d < 3; d++) {
+        lo[d] = w.s_lo[(size_t)d * cap + s];
+        hi[d] = w.s_hi[(size_t)d * cap + s];
+        mn[d] = d < dim ? dkey_inv(w.s_min[(size_t)d * cap + s]) : 0.0;
+        mx[d] = d < dim ? dkey_inv(w.s_max[(size_t)d * cap + s]) : 0.0;
+    }
+    int cut_dim, mode;
+    double cv;
+    kd_choose(lo, hi, mn, mx, dim, cut_dim, cv, mode);
     w.s_cd[s] = cut_dim;
     w.s_cv[s] = cv;
     w.s_mode[s] = mode;
@@ -510,7 +556,7 @@ __global__ void k_kd_br1(int nseg, KdWork w) {
     w.s_br1[s] = w.scan[e] - w.scan[b];
 }
 
-// n_lo rule (kd_split.cpp:208-212), node records and the next level.
+// Node records and the next level.
 __global__ void k_kd_children(int nseg, KdWork w, KdDev kd, const int *perm, int cap) {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nseg) return;
@@ -518,12 +564,11 @@ __global__ void k_kd_children(int nseg, KdWork w, KdDev kd, const int *perm, int
     int br1 = w.s_br1[s];
     int br2 = br1 + (w.scan[b + cnt] - w.scan[b + br1]);
     int mode = w.s_mode[s];
-    int n_lo;
-    if (mode == 1) n_lo = 1;
-    else if (mode == 2) n_lo = cnt - 1;
-    else if (br1 > cnt / 2) n_lo = br1;
-    else if (br2 < cnt / 2) n_lo = br2;
-    else n_lo = cnt / 2;
+    int n_lo = kd_n_lo(mode, cnt, br1, br2);
+    if (n_lo < 1 || n_lo >= cnt) {      // coordinates that do not compare (NaN)
+        w.counters[3] = 1;
+        n_lo = cnt / 2;
+    }
     w.s_nlo[s] = n_lo;
     int node = w.s_node[s];
     int cd = w.s_cd[s];
@@ -545,18 +590,20 @@ __global__ void k_kd_children(int nseg, KdWork w, KdDev kd, const int *perm, int
         if (cn == 1) {
             kd.leaf_of[perm[cstart]] = child;
         } else if (cn > 1) {
-            nseg_id = atomicAdd(&w.counters[0], 1);
-            w.n_start[nseg_id] = cstart;
-            w.n_n[nseg_id] = cn;
-            w.n_node[nseg_id] = child;
+            int at;
+            if (cn > KD_LOCAL) at = nseg_id = atomicAdd(&w.counters[0], 1);
+            else at = cap - 1 - atomicAdd(&w.counters[2], 1);
+            w.n_start[at] = cstart;
+            w.n_n[at] = cn;
+            w.n_node[at] = child;
             for (int d = 0; d < 3; d++) {
                 double lo = w.s_lo[(size_t)d * cap + s], hi = w.s_hi[(size_t)d * cap + s];
                 if (d == cd) {
                     if (side == 0) hi = cv;
                     else lo = cv;
                 }
-                w.n_lo[(size_t)d * cap + nseg_id] = lo;
-                w.n_hi[(size_t)d * cap + nseg_id] = hi;
+                w.n_lo[(size_t)d * cap + at] = lo;
+                w.n_hi[(size_t)d * cap + at] = hi;
             }
         }
         if (side == 0) w.s_clo[s] = nseg_id;
@@ -584,6 +631,140 @@ __global__ void k_kd_promote(int nseg, KdWork w, int cap) {
     }
 }
 
+// One workgroup splits one kept cell down to single points, level by level as
+// the kernels above do: thread p holds the point at position p of the cell,
+// the range [b, e) of its present sub-cell and that one's box and node.
+__global__ void __launch_bounds__(KD_LOCAL)
+k_kd_local(const double *__restrict__ pts, int n, int dim, KdWork w, KdDev kd, int cap) {
+    __shared__ double x[3][KD_LOCAL];                        // by place in the cell at the start
+    __shared__ unsigned long long s_mn[3][KD_LOCAL], s_mx[3][KD_LOCAL];   // by b
+    __shared__ int A[KD_LOCAL + 1], WL[KD_LOCAL], WR[KD_LOCAL], w_tot[KD_LOCAL / WAVE], s_base;
+    const int seg = cap - 1 - (int)blockIdx.x;
+    const int start = w.n_start[seg], m = w.n_n[seg];
+    const int p = threadIdx.x, lane = p & (WAVE - 1), wv = p / WAVE;
+    const bool live = p < m;
+    // exclusive prefix of a flag over the threads into A; the total
+    auto scan = [&](bool f) {
+        const unsigned long long h = __ballot(f);
+        if (lane == 0) w_tot[wv] = (int)__popcll(h);
+        __syncthreads();
+        int pre = 0, all = 0;
+        for (int u = 0; u < KD_LOCAL / WAVE; u++) {
+            if (u == wv) pre = all;
+            all += w_tot[u];
+        }
+        A[p] = pre + (int)__popcll(h & ((1ULL << lane) - 1ULL));
+        if (p == 0) A[KD_LOCAL] = all;
+        __syncthreads();
+        return all;
+    };
+    int id = p;                                              // place at the start of the point held now
+    const int g0 = live ? w.perm[start + p] : 0;             // its index
+    for (int d = 0; d < 3; d++) x[d][p] = live && d < dim ? pts[(size_t)d * n + g0] : 0.0;
+    int b = 0, e = m, node = w.n_node[seg];
+    int depth = kd.depth[node];
+    double lo[3], hi[3];
+    for (int d = 0; d < 3; d++) {
+        lo[d] = w.n_lo[(size_t)d * cap + seg];
+        hi[d] = w.n_hi[(size_t)d * cap + seg];
+    }
+    // a cell of m points has 2m - 2 nodes below its own
+    if (p == 0) s_base = atomicAdd(&w.counters[1], 2 * m - 2);
+    __syncthreads();
+    int base = s_base;
+    bool on = live && m > 1;
+    // every level splits every sub-cell of two or more points
+    while (__syncthreads_or(on)) {
+        if (on && p == b)
+            for (int d = 0; d < dim; d++) { s_mn[d][b] = ~0ULL; s_mx[d][b] = 0ULL; }
+        __syncthreads();
+        const int tag = on ? b : -1, up = __shfl_up(tag, 1, WAVE);
+        const bool head = on && (lane == 0 || up != tag);
+        for (int d = 0; d < dim; d++) {
+            unsigned long long mn = ~0ULL, mx = 0ULL;
+            if (on) mn = mx = dkey(x[d][id]);
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const unsigned long long on_ = __shfl_down(mn, o, WAVE), ox = __shfl_down(mx, o, WAVE);
+                const int ot = __shfl_down(tag, o, WAVE);
+                if (lane + o < WAVE && ot == tag) { mn = on_ < mn ? on_ : mn; mx = ox > mx ? ox : mx; }
+            }
+            if (head) {
+                atomicMin(&s_mn[d][b], mn);
+                atomicMax(&s_mx[d][b], mx);
+            }
+        }
+        __syncthreads();
+        int cd = 0, mode = 0;
+        double cv = 0.0;
+        if (on) {
+            double mn[3], mx[3];
+            for (int d = 0; d < 3; d++) {
+                mn[d] = d < dim ? dkey_inv(s_mn[d][b]) : 0.0;
+                mx[d] = d < dim ? dkey_inv(s_mx[d][b]) : 0.0;
+            }
+            kd_choose(lo, hi, mn, mx, dim, cd, cv, mode);
+        }
+        // annPlaneSplit's two passes: v < cv over the sub-cell, then v <= cv
+        // over what is left of it
+        int br[2] = {0, 0};
+        for (int pass = 0; pass < 2; pass++) {
+            const int from = b + (pass ? br[0] : 0);
+            const double v = on ? x[cd][id] : 0.0;
+            const bool f = on && p >= from && (pass ? v <= cv : v < cv);
+            scan(f);
+            const int C = on ? A[e] - A[from] : 0;
+            br[pass] = C;
+            const bool left = on && p >= from && p < from + C && !f, right = on && p >= from + C && f;
+            const int kl = left ? (p - from) - (A[p] - A[from]) : 0;
+            const int kr = right ? A[e] - A[p + 1] : 0;
+            if (left) WL[from + kl] = id;
+            if (right) WR[from + kr] = id;
+            __syncthreads();
+            if (left) id = WR[from + kl];
+            if (right) id = WL[from + kr];
+            __syncthreads();
+        }
+        int n_lo = on ? kd_n_lo(mode, e - b, br[0], br[0] + br[1]) : 0;
+        if (on && (n_lo < 1 || n_lo >= e - b)) {   // coordinates that do not compare (NaN)
+            w.counters[3] = 1;
+            n_lo = (e - b) / 2;
+        }
+        // two nodes for each sub-cell, in the order of the sub-cells
+        const bool lead = on && p == b;
+        const int segs = scan(lead);
+        if (on) {
+            const int c0 = base + 2 * A[b];
+            if (lead) {
+                kd.cd[node] = cd;
+                kd.cv[node] = cv;
+                for (int side = 0; side < 2; side++) {
+                    kd.parent[c0 + side] = node;
+                    kd.depth[c0 + side] = depth + 1;
+                    kd.is_hi[c0 + side] = side;
+                    kd.cd[c0 + side] = 0;
+                    kd.cv[c0 + side] = 0.0;
+                }
+            }
+            const int side = p - b >= n_lo ? 1 : 0;
+            node = c0 + side;
+            depth++;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+                if (d == cd) {
+                    if (side) lo[d] = cv;
+                    else hi[d] = cv;
+                }
+            if (side) b += n_lo;
+            else e = b + n_lo;
+            if (e - b == 1) {
+                kd.leaf_of[w.perm[start + id]] = node;
+                on = false;
+            }
+        }
+        base += 2 * segs;
+    }
+}
+
 void kd_build(hipStream_t st, const double *pts, int n, int dim, KdDev &kd, void *work, size_t work_bytes) {
     (void)work_bytes;
     KdWork w = carve(work, n);
@@ -596,10 +777,7 @@ void kd_build(hipStream_t st, const double *pts, int n, int dim, KdDev &kd, void
     hipLaunchKernelGGL(k_kd_init, dim3(gn), dim3(B), 0, st, n, w.perm, w.seg, kd);
     HIP_OK(hipMemsetAsync(w.counters, 0, sizeof(int) * 16, st));
     hipLaunchKernelGGL(k_kd_root, dim3(1), dim3(64), 0, st, d_bb, n, dim, w, kd, cap);
-    int nseg = n > 1 ? 1 : 0;
-    if (n <= 1) {
-        HIP_OK(hipMemsetAsync(w.seg, 0xFF, sizeof(int) * n, st));
-    }
+    int nseg = n > KD_LOCAL ? 1 : 0, local = n > 1 && n <= KD_LOCAL ? 1 : 0;
     int levels = 0;
     while (nseg > 0) {
         unsigned gs = (unsigned)((nseg + B - 1) / B);
@@ -620,19 +798,24 @@ void kd_build(hipStream_t st, const double *pts, int n, int dim, KdDev &kd, void
         HIP_OK(hipMemsetAsync(w.counters, 0, sizeof(int), st));
         hipLaunchKernelGGL(k_kd_children, dim3(gs), dim3(B), 0, st, nseg, w, kd, w.perm, cap);
         hipLaunchKernelGGL(k_kd_reseg, dim3(gn), dim3(B), 0, st, n, w.seg, w);
-        int next = 0;
-        HIP_OK(hipMemcpyAsync(&next, w.counters, sizeof(int), hipMemcpyDeviceToHost, st));
+        int cnt[3] = {0, 0, 0};
+        HIP_OK(hipMemcpyAsync(cnt, w.counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
+        const int next = cnt[0];
+        local = cnt[2];
         if (next > 0) {
             hipLaunchKernelGGL(k_kd_promote, dim3((unsigned)((next + B - 1) / B)), dim3(B), 0, st, next, w, cap);
         }
         nseg = next;
         if (++levels > n + 2) throw HipError("kd_build: no progress", hipErrorUnknown, __FILE__, __LINE__);
     }
-    int nodes = 0;
-    HIP_OK(hipMemcpyAsync(&nodes, w.counters + 1, sizeof(int), hipMemcpyDeviceToHost, st));
+    if (local > 0)
+        hipLaunchKernelGGL(k_kd_local, dim3((unsigned)local), dim3(KD_LOCAL), 0, st, pts, n, dim, w, kd, cap);
+    int bad = 0;
+    HIP_OK(hipMemcpyAsync(&bad, w.counters + 3, sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
-    kd.n_nodes = nodes;
+    if (bad) throw HipError("kd_build: no progress", hipErrorUnknown, __FILE__, __LINE__);
+    kd.n_nodes = 2 * n - 1;
     kd.valid = true;
 }
 
