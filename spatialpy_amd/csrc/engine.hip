@@ -49,6 +49,34 @@ template <class T> void d2h(hipStream_t s, T *dst, const T *src, size_t count) {
     if (count) HIP_OK(hipMemcpyAsync(dst, src, sizeof(T) * count, hipMemcpyDeviceToHost, s));
 }
 
+// Device memory of one call: one allocation for all of its arrays (an
+// allocation and its release cost tens of microseconds each).
+class Arena {
+  public:
+    Arena() = default;
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    ~Arena() {
+        if (base_) (void)hipFree(base_);
+    }
+    // f takes the arrays; it runs twice, first to add up their sizes
+    template <class F> void plan(F f) {
+        f(*this);
+        HIP_OK(hipMalloc((void **)&base_, std::max<size_t>(at_, 1)));
+        at_ = 0;
+        f(*this);
+    }
+    template <class T> T *take(size_t count) {
+        T *p = (T *)(base_ + at_);
+        at_ += (sizeof(T) * count + 255) & ~(size_t)255;
+        return p;
+    }
+
+  private:
+    char *base_ = nullptr;
+    size_t at_ = 0;
+};
+
 // component-major [3][n] <-> particle-major [n][3]
 std::vector<double> to_soa3(const double *aos, int n) {
     std::vector<double> o(3 * (size_t)n);
@@ -2569,73 +2597,107 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
                       int64_t *row_ptr, int32_t *idx, double *r2) {
     GUARD_BEGIN
     if (n <= 0 || m < 0 || dim < 1 || dim > 3 || !(h > 0)) return set_error(SSASDPD_ERR_BAD_DESC, "bad fr_search args");
-    hipStream_t st;
-    HIP_OK(hipStreamCreate(&st));
-    std::vector<double> hp = to_soa3(pts, n), hq = to_soa3(q, m);
-    double *dp = dalloc<double>(3 * (size_t)n), *dq = dalloc<double>(3 * (size_t)std::max(m, 1));
-    double *sp = dalloc<double>(4 * (size_t)n), *bb = dalloc<double>(8);
-    unsigned long long *bbt = dalloc<unsigned long long>(8);
-    int *srt = dalloc<int>(n), *cof = dalloc<int>(n);
-    h2d(st, dp, hp.data(), 3 * (size_t)n);
-    h2d(st, dq, hq.data(), 3 * (size_t)m);
+    // Everything up to the caller's arrays stays on the GPU: the points are
+    // laid out, the lists' lengths counted and scanned, and the rows written
+    // there.  The call with idx == NULL needs the lengths only.  (262,147
+    // points, 26 neighbours each: the two calls 72 -> 12.7 ms; the host had
+    // spent it on clearing and walking the column-major lists, on twenty
+    // allocations and on a second search where the first width was too small.)
+    hipStream_t st = hipStreamPerThread;
+    const int mq = std::max(m, 1);
+    Arena a;
+    double *stage = nullptr, *dp, *dq, *sp, *bb;
+    unsigned long long *bbt;
+    int *srt, *cof, *dg, *row32;
+    int64_t *row64;
+    DevErr *de;
+    a.plan([&](Arena &r) {
+        stage = r.take<double>(3 * (size_t)std::max(n, mq));
+        dp = r.take<double>(3 * (size_t)n);
+        dq = r.take<double>(3 * (size_t)mq);
+        sp = r.take<double>(4 * (size_t)n);
+        bb = r.take<double>(8);
+        bbt = r.take<unsigned long long>(8);
+        srt = r.take<int>(n);
+        cof = r.take<int>(n);
+        dg = r.take<int>(mq);
+        row32 = r.take<int>((size_t)mq + 1);
+        row64 = r.take<int64_t>((size_t)mq + 1);
+        de = r.take<DevErr>(1);
+    });
+    h2d(st, stage, pts, 3 * (size_t)n);
+    soa3(st, stage, n, dp);
+    if (m > 0) {
+        h2d(st, stage, q, 3 * (size_t)m);
+        soa3(st, stage, m, dq);
+    }
     compute_bbox(st, dp, n, dim, bb, bbt);
     double hb[6];
     d2h(st, hb, bb, 6);
     HIP_OK(hipStreamSynchronize(st));
     Grid g;
     grid_setup(hb, n, dim, h, g);
-    int *cc = dalloc<int>(g.ncell + 1), *cs = dalloc<int>(g.ncell + 2), *cf = dalloc<int>(g.ncell + 1);
-    void *stmp;
-    HIP_OK(hipMalloc(&stmp, std::max(scan_tmp_bytes(g.ncell + 8), scan_tmp_bytes(n + 8))));
+    Arena c;
+    int *cc, *cs, *cf;
+    char *stmp;
+    c.plan([&](Arena &r) {
+        cc = r.take<int>(g.ncell + 1);
+        cs = r.take<int>(g.ncell + 2);
+        cf = r.take<int>(g.ncell + 1);
+        stmp = r.take<char>(std::max(scan_tmp_bytes(g.ncell + 8), scan_tmp_bytes((size_t)std::max(n, mq) + 8)));
+    });
     bin_points(st, dp, n, dim, g, cof, cc, cs, cf, srt, sp, stmp);
     KdDev kd;
-    kd.parent = dalloc<int>(2 * (size_t)n + 2); kd.depth = dalloc<int>(2 * (size_t)n + 2);
-    kd.cd = dalloc<int>(2 * (size_t)n + 2); kd.cv = dalloc<double>(2 * (size_t)n + 2);
-    kd.is_hi = dalloc<int>(2 * (size_t)n + 2); kd.leaf_of = dalloc<int>(n);
-    size_t kws = kd_work_bytes(n);
-    void *kw;
-    HIP_OK(hipMalloc(&kw, kws));
-    kd_build(st, dp, n, dim, kd, kw, kws);
-    DevErr *de = dalloc<DevErr>(1);
-    int W = 16;
-    int *oi = nullptr, *dg = dalloc<int>(std::max(m, 1));
-    double *orr = nullptr;
-    for (int attempt = 0; attempt < 6; attempt++) {
-        dfree(oi); dfree(orr);
-        oi = dalloc<int>((size_t)W * std::max(m, 1));
-        orr = dalloc<double>((size_t)W * std::max(m, 1));
-        DevErr e0{0, INT32_MAX, 0, 0, 0};
+    Arena k;
+    // (the tree decides the order of a list, not its length; its build also
+    // refuses points that do not compare)
+    const bool nan = std::any_of(hb, hb + 2 * dim, [](double v) { return std::isnan(v); });
+    if (idx || nan) {
+        char *kw;
+        const size_t kws = kd_work_bytes(n), nodes = 2 * (size_t)n + 2;
+        k.plan([&](Arena &r) {
+            kd.parent = r.take<int>(nodes);
+            kd.depth = r.take<int>(nodes);
+            kd.cd = r.take<int>(nodes);
+            kd.cv = r.take<double>(nodes);
+            kd.is_hi = r.take<int>(nodes);
+            kd.leaf_of = r.take<int>(n);
+            kw = r.take<char>(kws);
+        });
+        kd_build(st, dp, n, dim, kd, kw, kws);
+    }
+    const DevErr e0{0, INT32_MAX, 0, 0, 0};
+    DevErr e = e0;
+    if (m > 0) {
         h2d(st, de, &e0, 1);
-        if (m > 0) fr_search(st, dq, m, sp, srt, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr);
-        DevErr e;
+        fr_count(st, dq, m, sp, cs, n, dim, h, g, dg, de);
+        exclusive_scan_i32(st, dg, row32, m, stmp);
+        rows64(st, row32, m, row64);
+        d2h(st, row_ptr, row64, (size_t)m + 1);
         d2h(st, &e, de, 1);
         HIP_OK(hipStreamSynchronize(st));
-        if (!e.overflow) break;
-        W = ((e.max_deg + 7) / 8) * 8 + 8;
+    } else {
+        row_ptr[0] = 0;
     }
-    std::vector<int> hd(std::max(m, 1));
-    d2h(st, hd.data(), dg, m);
-    HIP_OK(hipStreamSynchronize(st));
-    int64_t off = 0;
-    for (int i = 0; i < m; i++) { row_ptr[i] = off; off += hd[i]; }
-    row_ptr[m] = off;
-    if (idx) {
-        std::vector<int> hi((size_t)W * m);
-        std::vector<double> hr((size_t)W * m);
-        d2h(st, hi.data(), oi, (size_t)W * m);
-        d2h(st, hr.data(), orr, (size_t)W * m);
+    if (idx && m > 0 && row_ptr[m] > 0) {
+        const size_t tot = (size_t)row_ptr[m];
+        const int W = e.max_deg;
+        Arena l;
+        int *oi, *ci;
+        double *orr, *cr;
+        l.plan([&](Arena &r) {
+            oi = r.take<int>((size_t)W * m);
+            orr = r.take<double>((size_t)W * m);
+            ci = r.take<int>(tot);
+            cr = r.take<double>(tot);
+        });
+        fr_search(st, dq, m, sp, srt, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr, nullptr, W);
+        csr_lists(st, m, W, dg, row32, oi, orr, ci, cr);
+        d2h(st, idx, ci, tot);
+        if (r2) d2h(st, r2, cr, tot);
         HIP_OK(hipStreamSynchronize(st));
-        for (int i = 0; i < m; i++)
-            for (int k = 0; k < hd[i]; k++) {
-                idx[row_ptr[i] + k] = hi[(size_t)k * m + i];
-                r2[row_ptr[i] + k] = hr[(size_t)k * m + i];
-            }
     }
-    dfree(dp); dfree(dq); dfree(sp); dfree(bb); dfree(bbt); dfree(srt); dfree(cof); dfree(cc); dfree(cs); dfree(cf);
-    (void)hipFree(stmp); (void)hipFree(kw);
-    dfree(kd.parent); dfree(kd.depth); dfree(kd.cd); dfree(kd.cv); dfree(kd.is_hi); dfree(kd.leaf_of);
-    dfree(de); dfree(oi); dfree(orr); dfree(dg);
-    (void)hipStreamDestroy(st);
+    HIP_OK(hipStreamSynchronize(st));
     return 0;
     GUARD_END
 }

@@ -187,6 +187,14 @@ void fr_search(hipStream_t s, const double *q, int m, const double *spts, const 
                const int *cell_start, int n, int dim, double h, const Grid &g, const KdDev *kd,
                int W, int *out_idx, double *out_r2, int *deg, DevErr *err, const int *query_order,
                const FinishArgs *fin = nullptr, int slots_hint = 0);
+// the lists' lengths alone (deg, and the longest in err->max_deg)
+void fr_count(hipStream_t s, const double *q, int m, const double *spts, const int *cell_start, int n, int dim,
+              double h, const Grid &g, int *deg, DevErr *err);
+// [n][3] to [3][n]; row offsets to 64 bits (m + 1 of them); lists [W][m] to rows
+void soa3(hipStream_t s, const double *aos, int n, double *soa);
+void rows64(hipStream_t s, const int *row32, int m, int64_t *row64);
+void csr_lists(hipStream_t s, int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
+               double *cr);
 void kd_build(hipStream_t s, const double *pts, int n, int dim, KdDev &kd, void *work, size_t work_bytes);
 size_t kd_work_bytes(int n);
 size_t scan_tmp_bytes(long long n);

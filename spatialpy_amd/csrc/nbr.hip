@@ -316,8 +316,8 @@ static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // workgroup (k_kd_local), a point per thread.  A level over the whole array is
 // 27 launches and a wait for the host, about 100 us however small its cells
 // are, and a tree has some log2(n) + 4 levels: with the last ten of them in one
-// launch the tree of 64,000 points takes 0.6 instead of 1.9 ms, of 121 points
-// 0.04 instead of 0.7 ms.  1,024: the most a workgroup holds with a point per
+// launch the tree of 64,000 points takes 1.0 instead of 1.9 ms, of 121 points
+// 0.13 instead of 0.72 ms.  1,024: the most a workgroup holds with a point per
 // thread, at 85 KB of LDS.
 constexpr int KD_LOCAL = 1024;
 
@@ -888,14 +888,15 @@ __device__ __forceinline__ double edge_dij(double mi, double ri, double mj, doub
     return -2.0 * (mi * mj) / (mi + mj) * (ri + rj) / (ri * rj) * rr2 * wfd / (rr2 + 0.01 * h * h);
 }
 
+// SLOTS 0: the lists' lengths only.
 template <int SLOTS>
 __global__ void __launch_bounds__(WAVE)
 k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts, const int *__restrict__ sorted,
             const int *__restrict__ cell_start, int n, int dim, double h, Grid g, KdView kd, int W,
             int *__restrict__ out_idx, double *__restrict__ out_r2, int *__restrict__ deg, DevErr *err,
             const int *__restrict__ order, FinishArgs fin, int has_fin) {
-    __shared__ int l_idx[SLOTS * WAVE];
-    __shared__ double l_r2[SLOTS * WAVE];
+    __shared__ int l_idx[SLOTS > 0 ? SLOTS * WAVE : 1];
+    __shared__ double l_r2[SLOTS > 0 ? SLOTS * WAVE : 1];
     __shared__ double s_dm[FIN_MAX_DMAT];
     const int tl = (int)threadIdx.x;
     if (has_fin && fin.Ddiag) {
@@ -944,6 +945,10 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
                 nrow++;
             }
         auto accept = [&](int j, double dist) {
+            if constexpr (SLOTS == 0) {
+                cnt++;
+                return;
+            }
             if (cnt < L) {
                 LI(cnt) = j;
                 LD(cnt) = dist;
@@ -968,7 +973,7 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
                     const double2 *sp = (const double2 *)(spts + 4 * (size_t)p);
                     a[u] = sp[0];
                     b[u] = sp[1];
-                    jj[u] = sorted[p];
+                    jj[u] = SLOTS > 0 ? sorted[p] : 0;
                 }
 #pragma unroll
                 for (int u = 0; u < CB; u++) {
@@ -982,7 +987,9 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
                 }
             }
         }
-        if (cnt > W) {
+        if (SLOTS == 0) {
+            deg[qi] = cnt;
+        } else if (cnt > W) {
             atomicExch(&err->overflow, 1);
             deg[qi] = 0;
         } else {
@@ -1084,6 +1091,46 @@ void fr_search(hipStream_t s, const double *q, int m, const double *spts, const 
     else
         hipLaunchKernelGGL(k_fr_search<32>, grid, dim3(WAVE), 0, s, q, m, spts, sorted, cell_start, n, dim, h, g, v, W,
                            out_idx, out_r2, deg, err, order, f, hf);
+}
+
+void fr_count(hipStream_t s, const double *q, int m, const double *spts, const int *cell_start, int n, int dim,
+              double h, const Grid &g, int *deg, DevErr *err) {
+    hipLaunchKernelGGL(k_fr_search<0>, xcd_grid((m + WAVE - 1) / WAVE), dim3(WAVE), 0, s, q, m, spts, nullptr,
+                       cell_start, n, dim, h, g, KdView{}, 0, nullptr, nullptr, deg, err, nullptr, FinishArgs{}, 0);
+}
+
+// ---------------------------------------------------------------------------
+// Host layouts: particle-major points to component-major, 64-bit row offsets,
+// column-major lists to rows.
+__global__ void k_soa3(const double *aos, int n, double *soa) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    for (int d = 0; d < 3; d++) soa[(size_t)d * n + i] = aos[3 * (size_t)i + d];
+}
+__global__ void k_rows64(const int *row32, int m, int64_t *row64) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= m) row64[i] = row32[i];
+}
+__global__ void k_csr(int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
+                      double *cr) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m) return;
+    const int d = deg[i], o = row32[i];
+    for (int k = 0; k < d && k < W; k++) {
+        ci[o + k] = oi[(size_t)k * m + i];
+        cr[o + k] = orr[(size_t)k * m + i];
+    }
+}
+void soa3(hipStream_t s, const double *aos, int n, double *soa) {
+    if (n > 0) hipLaunchKernelGGL(k_soa3, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, aos, n, soa);
+}
+void rows64(hipStream_t s, const int *row32, int m, int64_t *row64) {
+    hipLaunchKernelGGL(k_rows64, dim3((unsigned)(((size_t)m + 256) / 256)), dim3(256), 0, s, row32, m, row64);
+}
+void csr_lists(hipStream_t s, int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
+               double *cr) {
+    if (m > 0)
+        hipLaunchKernelGGL(k_csr, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, m, W, deg, row32, oi, orr, ci, cr);
 }
 
 }  // namespace ssa

@@ -87,28 +87,7 @@ unsigned char *scratch_ptr() {
     return g_ptr[dev];
 }
 
-__global__ void k_na_soa(const double *aos, int n, double *soa) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    for (int d = 0; d < 3; d++) soa[(size_t)d * n + i] = aos[3 * (size_t)i + d];
-}
 
-__global__ void k_na_row64(const int *row32, int m, int64_t *row64) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i <= m) row64[i] = row32[i];
-}
-
-// ELL [W][m] -> CSR by the row offsets
-__global__ void k_na_csr(int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
-                         double *cr) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const int d = deg[i], o = row32[i];
-    for (int k = 0; k < d && k < W; k++) {
-        ci[o + k] = oi[(size_t)k * m + i];
-        cr[o + k] = orr[(size_t)k * m + i];
-    }
-}
 
 // Grid over the tree points' box with cell side >= h (every accepted pair
 // lies in neighbouring cells) and at most NA_MAX_CELLS cells.  The lists do
@@ -189,13 +168,12 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
         kd.cv = (double *)k; k += al(sizeof(double) * KD_NODES);
         kd.leaf_of = (int *)k;
     }
-    const unsigned B = 256;
     // points: host AoS -> staging -> SoA
     HIP_OK(hipMemcpyAsync(stage, pts, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_na_soa, dim3((n + B - 1) / B), dim3(B), 0, st, stage, n, dp);
+    soa3(st, stage, n, dp);
     if (m > 0) {
         HIP_OK(hipMemcpyAsync(stage, q, sizeof(double) * 3 * (size_t)m, hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_na_soa, dim3((m + B - 1) / B), dim3(B), 0, st, stage, m, dq);
+        soa3(st, stage, m, dq);
     }
     compute_bbox(st, dp, n, dim, bb, bbt);
     double hb[6];
@@ -225,12 +203,12 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
         return 0;
     }
     exclusive_scan_i32(st, dg, row32, m, stmp);
-    hipLaunchKernelGGL(k_na_row64, dim3((m + 1 + B - 1) / B), dim3(B), 0, st, row32, m, row64);
+    rows64(st, row32, m, row64);
     HIP_OK(hipMemcpyAsync(row_ptr, row64, sizeof(int64_t) * ((size_t)m + 1), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
     if (idx) {
         const size_t tot = (size_t)row_ptr[m];
-        hipLaunchKernelGGL(k_na_csr, dim3((m + B - 1) / B), dim3(B), 0, st, m, W, dg, row32, oi, orr, ci, cr);
+        csr_lists(st, m, W, dg, row32, oi, orr, ci, cr);
         HIP_OK(hipMemcpyAsync(idx, ci, sizeof(int) * tot, hipMemcpyDeviceToHost, st));
         if (r2) HIP_OK(hipMemcpyAsync(r2, cr, sizeof(double) * tot, hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
