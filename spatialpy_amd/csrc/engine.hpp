@@ -51,6 +51,30 @@ __device__ __forceinline__ int xcd_chunk(int nb) {
 }
 inline dim3 xcd_grid(int nb) { return dim3((unsigned)(((nb + N_XCD - 1) / N_XCD) * N_XCD)); }
 
+// A divisor that several quotients share.  For double: a Newton-refined
+// reciprocal, formed once, then per quotient one product and Markstein's
+// residual correction (q = a y, q + (a - b q) y).  With operands and quotients
+// in the normal range, as everywhere it is used, that is what an FP64 division
+// does on this hardware apart from its range scaling, so the quotient has the
+// same bits; 3 instructions instead of 11.  For float: the division.
+template <class R> struct Den {
+    R b;
+    __device__ __forceinline__ explicit Den(R d) : b(d) {}
+    __device__ __forceinline__ R div(R a) const { return a / b; }
+};
+template <> struct Den<double> {
+    double b, y;
+    __device__ __forceinline__ explicit Den(double d) : b(d) {
+        y = __builtin_amdgcn_rcp(d);
+        y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+        y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    }
+    __device__ __forceinline__ double div(double a) const {
+        const double q = a * y;
+        return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+    }
+};
+
 // Device-side error record.
 struct DevErr {
     int code;          // ssasdpd_status

@@ -885,6 +885,10 @@ __device__ __forceinline__ double edge_dij(double mi, double ri, double mj, doub
     double ihsq = ih * ih;
     double dhr = h - rr;
     double wfd = -25.066903536973515383e0 * dhr * dhr * ihsq * ihsq * ihsq * ih;
+    const double m = Den<double>(mi + mj).div(-2.0 * (mi * mj));
+    const double D = Den<double>(rr2 + 0.01 * h * h).div(Den<double>(ri * rj).div(m * (ri + rj)) * rr2 * wfd);
+    if (D == D) return D;
+    // a divisor of 0: the plain divisions tell inf and NaN apart
     return -2.0 * (mi * mj) / (mi + mj) * (ri + rj) / (ri * rj) * rr2 * wfd / (rr2 + 0.01 * h * h);
 }
 

@@ -15,6 +15,7 @@
 // reference with one thread reads it in index order (model.cpp:285-293).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "engine.hpp"
@@ -133,12 +134,27 @@ __global__ void __launch_bounds__(256) k_predict(SdpdArgs a) {
     for (int q = threadIdx.x; q < nrec * 8; q += 256) dst[q] = srec[q];
 }
 
+// The model's tables are the same for all lanes and never written by a kernel:
+// read through the constant address space they take scalar loads, also behind
+// a kernel's stores.
+__device__ __forceinline__ int tab_int(const int *p) { return *(const __attribute__((address_space(4))) int *)p; }
+__device__ __forceinline__ Rxn tab_rxn(const Rxn *p) {
+    Rxn r;
+    constexpr int N = sizeof(Rxn) / 4;
+    static_assert(sizeof(Rxn) % 4 == 0, "");
+    int w[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) w[k] = ((const __attribute__((address_space(4))) int *)p)[k];
+    __builtin_memcpy(&r, w, sizeof r);
+    return r;
+}
+
 // generated det<name> functions (solver.py:160-190), called with
 // vol = mass/rho and t = current_step*dt (model.cpp:181-184); VM: kind-4
 // rows through the expression VM (only k_chem instantiates it)
 template <bool VM>
 __device__ __forceinline__ double chem_rhs(const SdpdArgs &a, int i, int r) {
-    const Rxn &re = a.rx[r];
+    const Rxn re = tab_rxn(a.rx + r);
     if (re.mask && !((re.mask >> a.type[i]) & 1ULL)) return 0.0;
     const double *c = a.C + (size_t)i * a.Sc;
     if constexpr (VM) {
@@ -154,32 +170,89 @@ __device__ __forceinline__ double chem_rhs(const SdpdArgs &a, int i, int r) {
     }
 }
 
+// The particle this thread takes: the block's 256 particles in ascending order
+// of their degree.  A wavefront walks its lists as far as the longest of them,
+// 15 entries at 8.9 neighbours on average; with like degrees together the mean
+// over a block's four wavefronts is 8 to 10.  (Which thread takes a particle
+// decides nothing about its sums.)  Places past n count as degree 0.
+__device__ __forceinline__ int by_degree(const SdpdArgs &a, int base) {
+    constexpr int BINS = WAVE;
+    __shared__ int bin[BINS], order[256];
+    const int t = threadIdx.x;
+    if (t < BINS) bin[t] = 0;
+    __syncthreads();
+    const int k = base + t < a.n ? min(a.deg[base + t], BINS - 1) : 0;
+    const int at = atomicAdd(bin + k, 1);
+    __syncthreads();
+    if (t < BINS) {
+        const int c = bin[t];
+        int x = c;
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const int y = __shfl_up(x, o, WAVE);
+            if (t >= o) x += y;
+        }
+        bin[t] = x - c;
+    }
+    __syncthreads();
+    order[bin[k] + at] = t;
+    __syncthreads();
+    return base + order[t];
+}
+
+// 16 bytes per lane from global memory straight to LDS, lane l's at dst + 16 l
+// (no registers in between); dst is the same in every lane.
+__device__ __forceinline__ void to_lds16(const void *src, void *dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t *)src,
+                                     (__attribute__((address_space(3))) uint32_t *)dst, 16, 0, 0);
+}
+
 // pairwiseForce (model.cpp:39-191), list order.  Real = double is the
 // reference's arithmetic operation for operation; Real = float evaluates the
 // pair terms (kernel gradient, pressure, viscosity, background pressure,
 // transport tensor, continuity) in FP32 from FP64-formed differences dx, dv
 // and sums them into FP64 accumulators.  The species flux Q stays FP64.  For
-// static domains only Q is observable, so the momentum part is skipped.
+// static domains only Q is observable, so the momentum part is left out.
 // CHEM: the reaction fluxes are added here; otherwise k_chem adds them
 // afterwards (models with custom deterministic rates), to the same Q in the
 // same order.
-// SPECIES: the model has deterministic species (without them the species
-// flux and its registers drop out: more wavefronts hide the gathers).
-template <typename Real, bool CHEM, bool SPECIES = true>
+// NSC: room for the sums of that many deterministic species (the fields of the
+// first four are loaded an entry ahead).
+//
+// A lane sums its particle's list in order.  What bounds it is the FP64
+// arithmetic of two wavefronts per SIMD (204 registers: 350 FP64 instructions
+// an entry, 60% of the time at a million particles).  Three things kept it from
+// that: the longest list of a wavefront (see by_degree); 40 divisions by 8
+// different divisors (see Den); and the neighbours' records, one 128-byte line
+// each and 7 loads apiece, whose 64 lines per wavefront pushed each other out
+// of the 32 KB L1 between one load and the next (2.1 lines from L2 for each
+// record) and made every entry wait for its own gather.  Now eight lanes fetch
+// a record together, a line each time, straight to LDS, while the entry before
+// it is computed; piece c of record r stands at place c ^ (r & 7) of it, so
+// that 64 lanes reading one piece of their own records use all banks.
+// Measured (cylinder, FP64, 3 species): 0.53 -> 0.32 ms at 1,000,000
+// particles, 51 -> 37 us at 64,000.  Also tried, and slower: a lane per pair
+// with the terms summed through LDS (0.49 to 0.64 ms: the sums and the search
+// for a slot's particle cost more instructions than the idle lanes), and list
+// entries loaded two ahead (0.33 ms).
+template <typename Real, bool MOMENTUM, bool CHEM, int NSC>
 __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
+    constexpr int NR = MOMENTUM ? 256 : 1;
+    __shared__ char s_rec[NR * sizeof(PRec)];
+    __shared__ int s_j[NR];
     const int chunk = xcd_chunk((a.n + 255) / 256);
     if (chunk < 0) return;
-    int i = chunk * blockDim.x + threadIdx.x;
-    if (i >= a.n) return;
-    const size_t n = a.n;
+    const int i = by_degree(a, chunk * 256);
+    const bool mine = i < a.n;
+    const size_t n = a.n, ii = mine ? i : 0;
     const double h = a.h;
     const Real hR = (Real)a.h, P0 = (Real)a.P0, rho0 = (Real)a.rho0, alpha = (Real)a.alpha;
-    const double xi[3] = {a.x[i], a.x[n + i], a.x[2 * n + i]};
-    const double vi[3] = {a.v[i], a.v[n + i], a.v[2 * n + i]};
-    const double vti[3] = {a.vt[i], a.vt[n + i], a.vt[2 * n + i]};
+    const double xi[3] = {a.x[ii], a.x[n + ii], a.x[2 * n + ii]};
+    const double vi[3] = {a.v[ii], a.v[n + ii], a.v[2 * n + ii]};
+    const double vti[3] = {a.vt[ii], a.vt[n + ii], a.vt[2 * n + ii]};
     const Real viR[3] = {(Real)vi[0], (Real)vi[1], (Real)vi[2]};
     const Real dvti[3] = {(Real)(vi[0] - vti[0]), (Real)(vi[1] - vti[1]), (Real)(vi[2] - vti[2])};
-    const Real rhoi = (Real)a.rho[i], mi = (Real)a.mass[i], nui = (Real)a.nu[i];
+    const double rhoid = a.rho[ii], mid = a.mass[ii];
+    const Real rhoi = (Real)rhoid, mi = (Real)mid, nui = (Real)a.nu[ii];
     const Real Pi = P0 * (rhoi / rho0 - (Real)1.0);
     // the sums start where the predictor resets them (F = g, Fbp, Frho and
     // Q = 0: simulate.cpp:92-105), not from the arrays, so a second launch
@@ -187,36 +260,104 @@ __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
     double F[3] = {a.g[0], a.g[1], a.g[2]};
     double Fbp[3] = {0.0, 0.0, 0.0};
     double Frho = 0.0;
-    constexpr int MAXSC = 16;
-    double Q[SPECIES ? MAXSC : 1];
-    const int Sc = SPECIES ? (a.Sc < MAXSC ? a.Sc : MAXSC) : 0;
-    for (int s = 0; s < Sc; s++) Q[s] = 0.0;
-    const int ti = a.type[i];
-    const bool momentum = a.static_domain == 0;
-    const int dg = a.deg[i];
-    Real dx[3] = {0, 0, 0}, dv[3] = {0, 0, 0};
-    for (int k = 0; k < dg; k++) {
-        const size_t e = (size_t)k * n + i;
-        const int j = a.nidx[e];
-        const double rd = a.nr[e];
-        if (rd / h > 1.0) continue;
-        if (rd == 0.0) continue;
-        const Real r = (Real)rd;
-        const Real R = r / hR;
-        const Real dWdr = alpha * ((Real)-12 * r / (hR * hR)) * (((Real)1 - R) * ((Real)1 - R));
-        double xj[3], vj[3], vtj[3], nujd, rhojd, mjd;
-        double2 pmj = make_double2(0.0, 0.0);
-        if (momentum) {
-            load_rec(a.rec + j, xj, vj, vtj, nujd, rhojd, mjd);
-            pmj = load_rec_pm(a.rec + j);
+    constexpr bool SPECIES = NSC > 0;
+    constexpr int NS = SPECIES ? NSC : 1;
+    const int Sc = SPECIES ? min(a.Sc, NSC) : 0;
+    constexpr int NE = NS < 4 ? NS : 4;      // species whose fields are loaded ahead
+    double Q[NS], Ci[NE], Di[NE], Cj[NE];
+    const int ti = a.type[ii];
+    auto diffusion = [&](int s) {
+        const long long kk = (long long)a.Sc * (ti - 1) + s;   // type-major, model.cpp:163
+        return (kk < (long long)a.Sc * a.T) ? a.Dmat[kk] : 0.0;
+    };
+    for (int s = 0; s < NS; s++) Q[s] = 0.0;
+#pragma unroll
+    for (int s = 0; s < NE; s++) {
+        Ci[s] = Di[s] = Cj[s] = 0.0;
+        if (s < Sc) {
+            Di[s] = diffusion(s);
+            Ci[s] = a.C[ii * a.Sc + s];
+        }
+    }
+    const int dg = mine ? a.deg[ii] : 0;
+    const Den<Real> by_h(hR), by_hh(hR * hR);
+    const Den<double> by_hd(h), by_hhd(h * h);
+    const Real Pi_r = Pi / (rhoi * rhoi), inv_mi = (Real)1.0 / mi;
+
+    int longest = dg;
+    for (int o = 1; o < WAVE; o <<= 1) longest = max(longest, __shfl_xor(longest, o, WAVE));
+    longest = __builtin_amdgcn_readfirstlane(longest);
+    const int t = threadIdx.x & (WAVE - 1), wave = threadIdx.x & ~(WAVE - 1);
+    char *const recs = s_rec + (MOMENTUM ? wave * (int)sizeof(PRec) : 0);
+    int *const jrec = s_j + (MOMENTUM ? wave : 0);
+    // entry k of the lane's list: the particle and its distance (places past
+    // the end: the lane's own particle, which is skipped)
+    int j1 = 0;
+    double rd1 = 0.0;
+    auto entry = [&](int k) {
+        const size_t e = (size_t)k * n + ii;
+        j1 = k < dg ? a.nidx[e] : (int)ii;
+        rd1 = k < dg ? a.nr[e] : 0.0;
+    };
+    // the record of j1, without waiting for it
+    double2 rm = make_double2(1.0, 1.0);
+    const int piece = ((t & 7) ^ (t >> 3)) * 16;
+    auto gather = [&]() {
+        if constexpr (MOMENTUM) {
+            jrec[(t & 7) * 8 + (t >> 3)] = j1;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            int jr[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) jr[u] = jrec[(t >> 3) * 8 + u];
+#pragma unroll
+            for (int u = 0; u < 8; u++) to_lds16((const char *)(a.rec + jr[u]) + piece, recs + u * 1024);
         } else {
-            const double2 rm = load_rho_mass(a.rec + j);
+            rm = load_rho_mass(a.rec + j1);
+        }
+#pragma unroll
+        for (int s = 0; s < NE; s++)
+            if (s < Sc) Cj[s] = a.C[(size_t)j1 * a.Sc + s];
+    };
+    if (longest > 0) {
+        entry(0);
+        gather();
+    }
+    Real dx[3] = {0, 0, 0}, dv[3] = {0, 0, 0};
+    for (int k = 0; k < longest; k++) {
+        const double rd = rd1;
+        const int j = j1;
+        double xj[3], vj[3], vtj[3], nujd, rhojd, mjd, dC[NE];
+        double2 pmj = make_double2(0.0, 0.0);
+        if constexpr (MOMENTUM) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            auto at = [&](int u) { return *(const double2 *)(recs + t * 128 + ((u ^ (t & 7)) * 16)); };
+            const double2 a0 = at(0), a1 = at(1), a2 = at(2), a3 = at(3), a4 = at(4), a5 = at(5);
+            pmj = at(7);
+            xj[0] = a0.x; xj[1] = a0.y; xj[2] = a1.x;
+            vj[0] = a1.y; vj[1] = a2.x; vj[2] = a2.y;
+            vtj[0] = a3.x; vtj[1] = a3.y; vtj[2] = a4.x;
+            nujd = a4.y; rhojd = a5.x; mjd = a5.y;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        } else {
             rhojd = rm.x;
             mjd = rm.y;
         }
+#pragma unroll
+        for (int s = 0; s < NE; s++) dC[s] = Ci[s] - Cj[s];
+        if (k + 1 < longest) {
+            entry(k + 1);
+            gather();
+        }
+        const double Rd = by_hd.div(rd);
+        if (Rd > 1.0) continue;
+        if (rd == 0.0) continue;
+        const Real r = (Real)rd;
+        const Real R = by_h.div(r);
+        const Real dWdr = alpha * by_hh.div((Real)-12 * r) * (((Real)1 - R) * ((Real)1 - R));
         const Real rhoj = (Real)rhojd, mj = (Real)mjd;
-        const Real inv_rh = (Real)1.0 / (r + (Real)0.001 * hR);
-        if (momentum) {
+        const Den<Real> by_rh(r + (Real)0.001 * hR), by_rr(rhoi * rhoj);
+        const Real inv_rh = by_rh.div((Real)1.0);
+        if constexpr (MOMENTUM) {
             const Real nuj = (Real)nujd;
             Real dv_dx = 0;
             for (int d = 0; d < a.dim; d++) {
@@ -229,14 +370,13 @@ __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
             // P_j / rho_j^2 and m_j / rho_j from the record: the same
             // operations on the same values as here, done once per particle
             const Real Pj_r = (Real)pmj.x, mrj = (Real)pmj.y;
-            Real pg = Pi / (rhoi * rhoi) + Pj_r;
-            if (pg < 0) pg = -Pi / (rhoi * rhoi) + Pj_r;
-            const Real fp = (Real)-1.0 * mj * pg * dWdr / (r + (Real)0.001 * hR);
-            const Real fv = mj * ((Real)2.0 * (nui * nuj) / (nui + nuj)) * ((Real)1 / (r + (Real)0.001 * hR)) * dWdr /
-                            ((rhoi * rhoj));
+            Real pg = Pi_r + Pj_r;
+            if (pg < 0) pg = -Pi_r + Pj_r;
+            const Real fp = by_rh.div((Real)-1.0 * mj * pg * dWdr);
+            const Real fv = by_rr.div(mj * Den<Real>(nui + nuj).div((Real)2.0 * (nui * nuj)) * inv_rh * dWdr);
             const Real mri = mi / rhoi;
             const Real vsum = mri * mri + mrj * mrj;
-            const Real fbp = (Real)-10.0 * P0 * ((Real)1.0 / mi) * vsum * dWdr / (r + (Real)0.001 * hR);
+            const Real fbp = by_rh.div((Real)-10.0 * P0 * inv_mi * vsum * dWdr);
             Real ft[3];
             for (int p = 0; p < 3; p++) {
                 Real acc = 0;
@@ -244,7 +384,7 @@ __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
                 for (int q = 0; q < 3; q++)
                     Tp[q] = (Real)0.5 * ((rhoi * viR[p] * (-dvti[q])) + (rhoj * vjR[p] * (-dvtj[q])));
                 acc = Tp[0] * dx[0] + Tp[1] * dx[1] + Tp[2] * dx[2];
-                ft[p] = ((Real)1.0 / mi) * vsum * acc * dWdr / (r + (Real)0.001 * hR);
+                ft[p] = by_rh.div(inv_mi * vsum * acc * dWdr);
             }
             for (int d = 0; d < a.dim; d++) {
                 if (!a.skip_F) F[d] += (double)(fp * dx[d] + fv * dv[d] + ft[d]);
@@ -254,41 +394,53 @@ __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
             // multiplied by 0.0 there: for finite states it adds a signed
             // zero, which leaves the sum (which starts at +0) unchanged, so
             // it is not formed
-            Frho = Frho + (double)(rhoi * mrj * dv_dx * ((Real)1 / (r + (Real)0.001 * hR)) * dWdr -
+            Frho = Frho + (double)(rhoi * mrj * dv_dx * inv_rh * dWdr -
                                    mrj *
                                        (rhoi * (dvti[0] * dx[0] + dvti[1] * dx[1] + dvti[2] * dx[2]) +
                                         rhoj * (dvtj[0] * dx[0] + dvtj[1] * dx[1] + dvtj[2] * dx[2])) *
                                        inv_rh * dWdr);
         }
-        if (Sc > 0) {
-            const double Rd = rd / h;
-            const double dWdrd = a.alpha * (-12 * rd / (h * h)) * ((1 - Rd) * (1 - Rd));
-            const double rhoid = a.rho[i], mid = a.mass[i];
-            const double wfd = (1.0 / (rd + 0.001 * h)) * dWdrd;
-            const double dQc_base = 2.0 * ((mid * mjd) / (mid + mjd)) * ((rhoid + rhojd) / (rhoid * rhojd)) *
-                                    (rd * rd) * wfd / ((rd * rd) + 0.01 * h * h);
-            for (int s = 0; s < Sc; s++) {
-                const long long kk = (long long)a.Sc * (ti - 1) + s;   // type-major, model.cpp:163
-                const double D = (kk < (long long)a.Sc * a.T) ? a.Dmat[kk] : 0.0;
-                Q[s] += D * (a.C[(size_t)i * a.Sc + s] - a.C[(size_t)j * a.Sc + s]) * dQc_base;
+        if constexpr (SPECIES) {
+            const double dWdrd = a.alpha * by_hhd.div(-12 * rd) * ((1 - Rd) * (1 - Rd));
+            double inv_rhd, rsum;
+            if constexpr (sizeof(Real) == 8) {
+                inv_rhd = inv_rh;
+                rsum = by_rr.div(rhoid + rhojd);
+                if (rsum != rsum) rsum = (rhoid + rhojd) / (rhoid * rhojd);   // a density of 0
+            } else {
+                inv_rhd = Den<double>(rd + 0.001 * h).div(1.0);
+                rsum = (rhoid + rhojd) / (rhoid * rhojd);
             }
+            const double wfd = inv_rhd * dWdrd;
+            const double dQc_base = Den<double>((rd * rd) + 0.01 * h * h)
+                                        .div(2.0 * Den<double>(mid + mjd).div(mid * mjd) * rsum * (rd * rd) * wfd);
+#pragma unroll
+            for (int s = 0; s < NE; s++)
+                if (s < Sc) Q[s] += Di[s] * dC[s] * dQc_base;
+            for (int s = NE; s < Sc; s++)
+                Q[s] += diffusion(s) * (a.C[ii * a.Sc + s] - a.C[(size_t)j * a.Sc + s]) * dQc_base;
         }
     }
+    if (!mine) return;
     if constexpr (CHEM) {
         for (int r = 0; r < a.Rc; r++) {
             const double flux = chem_rhs<false>(a, i, r);
-            for (int s = 0; s < Sc; s++) {
-                const long long kk = (long long)a.Rc * r + s;             // model.cpp:186
-                const int nk = kk < (long long)a.Sc * a.Rc ? a.Ndense[kk] : 0;
-                Q[s] += nk * flux;
-            }
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+                if (s < Sc) {
+                    const long long kk = (long long)a.Rc * r + s;             // model.cpp:186
+                    const int nk = kk < (long long)a.Sc * a.Rc ? tab_int(a.Ndense + kk) : 0;
+                    Q[s] += nk * flux;
+                }
         }
     }
-    if (momentum) {
+    if constexpr (MOMENTUM) {
         for (int d = 0; d < 3; d++) { a.F[d * n + i] = F[d]; a.Fbp[d * n + i] = Fbp[d]; }
         a.Frho[i] = Frho;
     }
-    for (int s = 0; s < Sc; s++) a.Q[(size_t)i * a.Sc + s] = Q[s];
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+        if (s < Sc) a.Q[(size_t)i * a.Sc + s] = Q[s];
 }
 
 __device__ __forceinline__ double cube(double x) { return x * x * x; }
@@ -419,21 +571,24 @@ __global__ void __launch_bounds__(256) k_chem(SdpdArgs a) {
     }
 }
 
+template <bool CHEM, int NSC> static void forces_as(hipStream_t s, const SdpdArgs &a) {
+    const dim3 g = grid1(a.n), b(256);
+    if (a.static_domain) {
+        if constexpr (NSC > 0) hipLaunchKernelGGL((k_forces<double, false, CHEM, NSC>), g, b, 0, s, a);
+    } else if (a.fp32) {
+        hipLaunchKernelGGL((k_forces<float, true, CHEM, NSC>), g, b, 0, s, a);
+    } else {
+        hipLaunchKernelGGL((k_forces<double, true, CHEM, NSC>), g, b, 0, s, a);
+    }
+}
 void sdpd_forces(hipStream_t s, const SdpdArgs &a) {
-    const bool vm = a.vm_code != nullptr && a.Rc > 0 && a.Sc > 0;
-    if (vm) {
-        if (a.fp32) hipLaunchKernelGGL((k_forces<float, false>), grid1(a.n), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_forces<double, false>), grid1(a.n), dim3(256), 0, s, a);
-        hipLaunchKernelGGL(k_chem, grid1(a.n), dim3(256), 0, s, a);
-        return;
-    }
-    if (a.Sc == 0) {
-        if (a.fp32) hipLaunchKernelGGL((k_forces<float, false, false>), grid1(a.n), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_forces<double, false, false>), grid1(a.n), dim3(256), 0, s, a);
-        return;
-    }
-    if (a.fp32) hipLaunchKernelGGL((k_forces<float, true>), grid1(a.n), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_forces<double, true>), grid1(a.n), dim3(256), 0, s, a);
+    const bool vm = a.vm_code != nullptr && a.Rc > 0;
+    if (a.Sc == 0) forces_as<false, 0>(s, a);
+    else if (vm && a.Sc <= 4) forces_as<false, 4>(s, a);
+    else if (vm) forces_as<false, 16>(s, a);
+    else if (a.Sc <= 4) forces_as<true, 4>(s, a);
+    else forces_as<true, 16>(s, a);
+    if (vm && a.Sc > 0) hipLaunchKernelGGL(k_chem, grid1(a.n), dim3(256), 0, s, a);
 }
 void sdpd_correct(hipStream_t s, const SdpdArgs &a) {
     if (!a.static_domain) hipLaunchKernelGGL(k_correct, grid1(a.n), dim3(256), 0, s, a);
