@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "engine.hpp"
+#include "download.hpp"
 #include "vm.hpp"
 #include "mpn.hpp"
 
@@ -113,9 +114,16 @@ struct ssasdpd_engine {
     double g[3] = {0, 0, 0};
     std::vector<uint32_t> out_steps;
     // initial state (host)
-    std::vector<double> x0, v0, rho0v, C0;
     std::vector<uint32_t> u0;
-    std::vector<double> nu0;
+    // the state a reset starts from, on the device (an upload of it was 13 ms
+    // of each run at a million particles): x, v, rho, nu, C, xx, and what a
+    // renumber permutes; one allocation
+    char *init = nullptr;
+    size_t i_x = 0, i_v = 0, i_rho = 0, i_nu = 0, i_C = 0, i_xx = 0, i_mass = 0, i_type = 0, i_solid = 0, i_dfn = 0,
+           i_perm = 0;
+    template <class T> void from_init(T *dst, size_t at, size_t count) {
+        if (count) HIP_OK(hipMemcpyAsync(dst, init + at, sizeof(T) * count, hipMemcpyDeviceToDevice, st));
+    }
 
     hipStream_t st = nullptr;
     // particles
@@ -236,6 +244,7 @@ struct ssasdpd_engine {
     ssasdpd_stats stats{};
     int max_deg_seen = 0;
     int last_max_deg = 0;       // longest list of the last search
+    PinnedRing ring;         // results on their way to the caller
     // Particle renumbering (moving domains, seeded mode): every
     // RENUMBER_EVERY steps the particles are put in cell order, so that
     // neighbours in space are neighbours in memory.  perm[p] is the caller's
@@ -258,8 +267,7 @@ struct ssasdpd_engine {
     }
     void *pbuf = nullptr, *stage = nullptr;
     size_t pbuf_cap = 0, stage_cap = 0;
-    std::vector<double> mass_h, dfn_h;
-    std::vector<int> type_h, solid_h;
+    std::vector<int> solid_h;
     // GPU time per phase, HIP events on the engine stream: 0 binning + tree,
     // 1 search + D_ij, 2 SDPD substeps, 3 rates + queue build, 4 SSA loop,
     // 5 force kernel alone
@@ -344,6 +352,8 @@ struct ssasdpd_engine {
         dfree(rtype); dfree(rmap); dfree(xbuf); dfree(Ddiag_alt); dfree(vol_alt);
         if (ps) (void)hipStreamDestroy(ps);
         ps = nullptr;
+        ring.release();
+        dfree(init);
         dfree(xtree); dfree(spts); dfree(d_bbox); dfree(d_bbtmp); dfree(rec);
         if (h_bbox) (void)hipHostFree(h_bbox);
         h_bbox = nullptr;
@@ -571,9 +581,7 @@ struct ssasdpd_engine {
         std::vector<int> ty(d->type, d->type + n), so(d->fixed, d->fixed + n);
         h2d(st, type, ty.data(), n);
         h2d(st, solid, so.data(), n);
-        type_h = ty;
         solid_h = so;
-        mass_h.assign(d->mass, d->mass + n);
         perm = dalloc<int>(n);
         perm_tmp = dalloc<int>(n);
         perm_h.resize(n);
@@ -601,14 +609,36 @@ struct ssasdpd_engine {
         for (int i = 0; i < n; i++)
             if (!so[i]) movers.push_back(i);
         h2d(st, mass, d->mass, n);
-        x0 = to_soa3(d->x, n);
-        v0 = to_soa3(d->v, n);
-        rho0v.assign(d->rho, d->rho + n);
-        nu0.assign(d->nu, d->nu + n);
+        const std::vector<double> x0 = to_soa3(d->x, n), v0 = to_soa3(d->v, n);
         if (S > 0) u0.assign(d->u0, d->u0 + (size_t)n * S);
-        C0.assign((size_t)n * Sc, 0.0);
+        std::vector<double> C0((size_t)n * Sc, 0.0);
         for (size_t k = 0; k < (size_t)n * Sc; k++)
             C0[k] = d->C0 ? d->C0[k] : (S == Sc && d->u0 ? (double)d->u0[k] : 0.0);
+        {
+            size_t at = 0;
+            auto room = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
+            const size_t nn = n, dfs = std::max(d->n_data_fn, 0);
+            i_x = room(24 * nn); i_v = room(24 * nn); i_rho = room(8 * nn); i_nu = room(8 * nn);
+            i_C = room(8 * nn * Sc); i_xx = room(4 * nn * S); i_mass = room(8 * nn); i_type = room(4 * nn);
+            i_solid = room(4 * nn); i_dfn = room(8 * nn * dfs); i_perm = room(4 * nn);
+            init = dalloc<char>(at);
+            h2d(st, (double *)(init + i_x), x0.data(), 3 * nn);
+            h2d(st, (double *)(init + i_v), v0.data(), 3 * nn);
+            h2d(st, (double *)(init + i_rho), d->rho, nn);
+            h2d(st, (double *)(init + i_nu), d->nu, nn);
+            h2d(st, (double *)(init + i_C), C0.data(), nn * Sc);
+            h2d(st, (uint32_t *)(init + i_xx), u0.data(), nn * S);
+            if (dfs) h2d(st, (double *)(init + i_dfn), d->data_fn, nn * dfs);
+            auto keep = [&](size_t o, const void *src, size_t bytes) {
+                HIP_OK(hipMemcpyAsync(init + o, src, bytes, hipMemcpyDeviceToDevice, st));
+            };
+            keep(i_mass, mass, 8 * nn);
+            keep(i_type, type, 4 * nn);
+            keep(i_solid, solid, 4 * nn);
+            keep(i_perm, perm, 4 * nn);
+            // the uploads read x0, v0 and C0
+            HIP_OK(hipStreamSynchronize(st));
+        }
         int Smax = std::max(S, Sc), Rmax = std::max(R, Rc);
         if (Smax > 0 && d->diffusion_matrix) {
             Dmat = dalloc<double>((size_t)Smax * T);
@@ -635,7 +665,6 @@ struct ssasdpd_engine {
             n_df = d->n_data_fn;
             dfn = dalloc<double>((size_t)n * n_df);
             h2d(st, dfn, d->data_fn, (size_t)n * n_df);
-            dfn_h.assign(d->data_fn, d->data_fn + (size_t)n * n_df);
         }
         if (R > 0) {
             int nnz = d->jcN[R];
@@ -689,34 +718,32 @@ qwork = dalloc<char>(q_work_bytes(n));
         size_t n3 = 3 * (size_t)n;
         if (renumbered) {
             // the constant per-particle arrays back in the caller's numbering
-            h2d(st, mass, mass_h.data(), n);
-            h2d(st, type, type_h.data(), n);
-            h2d(st, solid, solid_h.data(), n);
-            if (n_df > 0) h2d(st, dfn, dfn_h.data(), (size_t)n * n_df);
-            for (int i = 0; i < n; i++) perm_h[i] = i;
-            h2d(st, perm, perm_h.data(), n);
+            from_init(mass, i_mass, n);
+            from_init(type, i_type, n);
+            from_init(solid, i_solid, n);
+            if (n_df > 0) from_init(dfn, i_dfn, (size_t)n * n_df);
+            from_init(perm, i_perm, n);
             renumbered = false;
-            perm_h_stale = false;
-            rebuild_movers();
+            perm_h_stale = movers_stale = true;
         }
-        h2d(st, x, x0.data(), n3);
-        h2d(st, v, v0.data(), n3);
+        from_init(x, i_x, n3);
+        from_init(v, i_v, n3);
         HIP_OK(hipMemsetAsync(vt, 0, sizeof(double) * n3, st));
         HIP_OK(hipMemsetAsync(F, 0, sizeof(double) * n3, st));
         HIP_OK(hipMemsetAsync(Fbp, 0, sizeof(double) * n3, st));
         HIP_OK(hipMemsetAsync(normal, 0, sizeof(double) * n3, st));
-        h2d(st, rho, rho0v.data(), n);
-        h2d(st, old_rho, rho0v.data(), n);
-        h2d(st, nu, nu0.data(), n);
+        from_init(rho, i_rho, n);
+        from_init(old_rho, i_rho, n);
+        from_init(nu, i_nu, n);
         HIP_OK(hipMemsetAsync(Frho, 0, sizeof(double) * n, st));
         HIP_OK(hipMemsetAsync(bvf, 0, sizeof(double) * n, st));
         if (Sc > 0) {
-            h2d(st, C, C0.data(), (size_t)n * Sc);
+            from_init(C, i_C, (size_t)n * Sc);
             HIP_OK(hipMemsetAsync(Q, 0, sizeof(double) * n * Sc, st));
         }
         HIP_OK(hipMemsetAsync(deg, 0, sizeof(int) * n, st));
         if (S > 0) {
-            h2d(st, xx, u0.data(), (size_t)n * S);
+            from_init(xx, i_xx, (size_t)n * S);
             HIP_OK(hipMemsetAsync(srrate, 0, sizeof(double) * n, st));
             HIP_OK(hipMemsetAsync(sdrate, 0, sizeof(double) * n, st));
             QueueState q{};
@@ -1371,7 +1398,13 @@ qwork = dalloc<char>(q_work_bytes(n));
         b_init.assign(B, 0);
         h2d(st, b_seeds, (const unsigned long long *)seeds, B);
         const size_t nn = n;
-        for (int b = 0; b < B; b++) h2d(st, b_xx + (size_t)b * nn * S, u0.data(), nn * S);
+        // every trajectory's counts: the first from the reset, then twice as
+        // many with each copy
+        if (S > 0) HIP_OK(hipMemcpyAsync(b_xx, xx, sizeof(uint32_t) * nn * S, hipMemcpyDeviceToDevice, st));
+        for (size_t have = 1; S > 0 && have < (size_t)B; have *= 2)
+            HIP_OK(hipMemcpyAsync(b_xx + have * nn * S, b_xx,
+                                  sizeof(uint32_t) * nn * S * std::min(have, (size_t)B - have),
+                                  hipMemcpyDeviceToDevice, st));
         HIP_OK(hipMemsetAsync(b_sr, 0, sizeof(double) * nn * B, st));
         HIP_OK(hipMemsetAsync(b_sd, 0, sizeof(double) * nn * B, st));
         std::vector<QueueState> q0(B);
@@ -1439,27 +1472,20 @@ qwork = dalloc<char>(q_work_bytes(n));
     }
 
     void snapshot(ssasdpd_outputs *o, int k) {
-        size_t nn = n;
-        std::vector<double> tmp;
-        if (o->xx && S > 0) d2h(st, o->xx + (size_t)k * nn * S, orig(xx, S), nn * S);
-        if (o->C && Sc > 0) d2h(st, o->C + (size_t)k * nn * Sc, orig(C, Sc), nn * Sc);
-        if (o->rho) d2h(st, o->rho + (size_t)k * nn, orig(rho, 1), nn);
-        if (o->bvf_phi) d2h(st, o->bvf_phi + (size_t)k * nn, orig(bvf, 1), nn);
-        if (o->nu) d2h(st, o->nu + (size_t)k * nn, orig(nu, 1), nn);
-        if (o->x) {
-            tmp.resize(3 * nn);
-            d2h(st, tmp.data(), orig3(x), 3 * nn);
-            HIP_OK(hipStreamSynchronize(st));
-            from_soa3(tmp, o->x + (size_t)k * nn * 3, n);
-        }
-        if (o->v) {
-            tmp.resize(3 * nn);
-            d2h(st, tmp.data(), orig3(v), 3 * nn);
-            HIP_OK(hipStreamSynchronize(st));
-            from_soa3(tmp, o->v + (size_t)k * nn * 3, n);
-        }
+        const size_t nn = n;
+        const bool xx_ = o->xx && S > 0, C_ = o->C && Sc > 0;
+        Download out(st, ring, nn * ((xx_ ? 4 * (size_t)S : 0) +
+                                     8 * ((C_ ? (size_t)Sc : 0) + (o->rho ? 1 : 0) + (o->bvf_phi ? 1 : 0) +
+                                          (o->nu ? 1 : 0) + (o->x ? 3 : 0) + (o->v ? 3 : 0))));
+        if (xx_) out.put(o->xx + (size_t)k * nn * S, orig(xx, S), nn * S);
+        if (C_) out.put(o->C + (size_t)k * nn * Sc, orig(C, Sc), nn * Sc);
+        if (o->rho) out.put(o->rho + (size_t)k * nn, orig(rho, 1), nn);
+        if (o->bvf_phi) out.put(o->bvf_phi + (size_t)k * nn, orig(bvf, 1), nn);
+        if (o->nu) out.put(o->nu + (size_t)k * nn, orig(nu, 1), nn);
+        if (o->x) out.put3(o->x + (size_t)k * nn * 3, orig3(x), nn);
+        if (o->v) out.put3(o->v + (size_t)k * nn * 3, orig3(v), nn);
         if (o->steps) o->steps[k] = cur;
-        HIP_OK(hipStreamSynchronize(st));
+        out.finish();
     }
 };
 
@@ -1790,8 +1816,11 @@ int ssasdpd_run(ssasdpd_engine *e, const ssasdpd_rng *r, ssasdpd_outputs *o) {
             uint32_t *d_xx = (K > 0 && o->xx) ? dalloc<uint32_t>(per * K) : nullptr;
             e->ssa_fused(e->rdme_args(step), 1, e->nt, sst, d_xx, 0, nullptr);
             rc = e->check(e->nt - 1);
-            for (int j = 0; j < K && !rc; j++)
-                if (d_xx) d2h(e->st, o->xx + (size_t)ks[j] * per, d_xx + (size_t)j * per, per);
+            if (d_xx && !rc) {
+                Download out(e->st, e->ring, sizeof(uint32_t) * per * K);
+                for (int j = 0; j < K; j++) out.put(o->xx + (size_t)ks[j] * per, d_xx + (size_t)j * per, per);
+                out.finish();
+            }
             HIP_OK(hipStreamSynchronize(e->st));
             dfree(d_xx);
             if (rc) return rc;
@@ -1845,9 +1874,10 @@ int ssasdpd_run_batch(ssasdpd_engine *e, int32_t n_traj, const uint64_t *seeds, 
     auto snap = [&](int k) {
         snap_shared(k, e->cur);
         if (counts && e->S > 0) {
+            Download out(e->st, e->ring, sizeof(uint32_t) * per * B);
             for (int b = 0; b < B; b++)
-                d2h(e->st, counts + ((size_t)b * n_snap + k) * per, e->orig(e->b_xx + (size_t)b * per, e->S), per);
-            HIP_OK(hipStreamSynchronize(e->st));
+                out.put(counts + ((size_t)b * n_snap + k) * per, e->orig(e->b_xx + (size_t)b * per, e->S), per);
+            out.finish();
         }
     };
     uint32_t next = 0;
@@ -1883,10 +1913,12 @@ int ssasdpd_run_batch(ssasdpd_engine *e, int32_t n_traj, const uint64_t *seeds, 
             uint32_t *d_xx = (counts && e->S > 0) ? dalloc<uint32_t>(per * K * B) : nullptr;
             e->ssa_fused(e->batch_args(step), B, e->nt, sst, d_xx, per * K, nullptr);
             rc = e->batch_check(B, e->nt - 1);
-            for (int j = 0; j < K && !rc; j++) {
-                if (d_xx)
-                    for (int b = 0; b < B; b++)
-                        d2h(e->st, counts + ((size_t)b * n_snap + ks[j]) * per, d_xx + ((size_t)b * K + j) * per, per);
+            if (d_xx && !rc) {
+                Download out(e->st, e->ring, sizeof(uint32_t) * per * K * B);
+                for (int b = 0; b < B; b++)
+                    for (int j = 0; j < K; j++)
+                        out.put(counts + ((size_t)b * n_snap + ks[j]) * per, d_xx + ((size_t)b * K + j) * per, per);
+                out.finish();
             }
             HIP_OK(hipStreamSynchronize(e->st));
             dfree(d_xx);
@@ -2508,33 +2540,31 @@ int ssasdpd_get_state(ssasdpd_engine *e, ssasdpd_state *s) {
     GUARD_BEGIN
     const int n = e->n;
     hipStream_t st = e->st;
-    std::vector<double> tmp(3 * (size_t)n);
     // every array in the caller's numbering
+    size_t total = 0;
+    for (const double *p : {s->x, s->v, s->vt, s->F, s->Fbp}) total += p ? 24 : 0;
+    for (const double *p : {s->rho, s->Frho, s->bvf_phi, s->nu, s->old_rho}) total += p ? 8 : 0;
+    total += 8 * (size_t)e->Sc * ((s->C ? 1 : 0) + (s->Q ? 1 : 0)) +
+             (size_t)e->S * ((s->xx ? 4 : 0) + (s->Ddiag ? 8 : 0)) + (s->rrate ? 8 * (size_t)e->R : 0);
+    Download out(st, e->ring, (size_t)n * total);
     auto v3 = [&](double *dst, double *src) {
-        if (!dst) return;
-        d2h(st, tmp.data(), e->orig3(src), 3 * (size_t)n);
-        HIP_OK(hipStreamSynchronize(st));
-        from_soa3(tmp, dst, n);
+        if (dst) out.put3(dst, e->orig3(src), n);
     };
     v3(s->x, e->x); v3(s->v, e->v); v3(s->vt, e->vt); v3(s->F, e->F); v3(s->Fbp, e->Fbp);
-    auto v1 = [&](double *dst, double *src, int cols) {
-        if (dst && src) {
-            d2h(st, dst, e->orig(src, cols), (size_t)n * cols);
-            HIP_OK(hipStreamSynchronize(st));
-        }
+    auto v1 = [&](auto *dst, auto *src, int cols) {
+        if (dst && src) out.put(dst, e->orig(src, cols), (size_t)n * cols);
     };
     v1(s->rho, e->rho, 1); v1(s->Frho, e->Frho, 1); v1(s->bvf_phi, e->bvf, 1); v1(s->nu, e->nu, 1);
     v1(s->old_rho, e->old_rho, 1);
     if (e->Sc) { v1(s->C, e->C, e->Sc); v1(s->Q, e->Q, e->Sc); }
     if (e->S) {
-        if (s->xx) d2h(st, s->xx, e->orig(e->xx, e->S), (size_t)n * e->S);
-        HIP_OK(hipStreamSynchronize(st));
+        v1(s->xx, e->xx, e->S);
         v1(s->srrate, e->srrate, 1); v1(s->sdrate, e->sdrate, 1);
         if (e->R) v1(s->rrate, e->rrate, e->R);
         v1(s->Ddiag, e->Ddiag, e->S);
         v1(s->next_time, e->qtime, 1);
     }
-    HIP_OK(hipStreamSynchronize(st));
+    out.finish();
     return 0;
     GUARD_END
 }
