@@ -342,11 +342,13 @@ __global__ void __launch_bounds__(256) k_ecn_infer(EcnGraph g, EcnScales s, cons
 // Y[M][N] = act(A[M][K] W[K][N] + bias) with Wt: bf16 [N][K] (the weights
 // transposed); Z (optional) receives the pre-activation.  A is FP32 and
 // enters as bf16 hi + lo halves.  K % 32 == 0, N % 16 == 0, N <= 64, K <= 64.
-// One wavefront computes 16 rows x all N columns.
+// One wavefront computes 16 rows x all N columns.  Zin (optional): Y is the
+// product times hs'(Zin), the backward pass through an activation.
 template <int N>
 __global__ void __launch_bounds__(256) k_gemm(int M, int K, const float *__restrict__ A, int lda,
                                               const __bf16 *__restrict__ Wt, const float *__restrict__ bias, int act,
-                                              float *__restrict__ Z, float *__restrict__ Y, int ldy) {
+                                              float *__restrict__ Z, float *__restrict__ Y, int ldy,
+                                              const float *__restrict__ Zin) {
     __shared__ __align__(16) __bf16 wsh[N * 64];
     for (int i = threadIdx.x; i < N * K; i += blockDim.x) wsh[i] = Wt[i];
     __syncthreads();
@@ -387,6 +389,7 @@ __global__ void __launch_bounds__(256) k_gemm(int M, int K, const float *__restr
             float z = acc[t][i];
             if (bias) z += bias[col];
             if (Z) Z[(size_t)r * N + col] = z;
+            if (Zin) z *= hsw_grad(Zin[(size_t)r * N + col]);
             Y[(size_t)r * ldy + col] = act ? hsw(z) : z;
         }
     }
@@ -395,21 +398,21 @@ __global__ void __launch_bounds__(256) k_gemm(int M, int K, const float *__restr
 // part[block][K][N] = A^T dY over the block's 64 rows: bf16 operands
 // staged in LDS, FP32 accumulation.  k_sum_parts adds the blocks' partials
 // in block order, so the gradient does not depend on scheduling.  K, N
-// multiples of 16 and <= 64.
+// multiples of 16 and <= 64.  132,864 rows, K = 64: 40 -> 33 us with padded rows.
 template <int N>
 __global__ void __launch_bounds__(256) k_gemm_wgrad(int M, int K, const float *__restrict__ A, int lda,
                                                     const float *__restrict__ dY, int ldy, float *__restrict__ part) {
-    constexpr int RB = 64;
-    __shared__ __align__(16) __bf16 at[64 * RB];   // A^T chunk [k][row]
-    __shared__ __align__(16) __bf16 dt[N * RB];    // dY^T chunk [n][row]
+    constexpr int RB = 64, RP = RB + 8;            // rows, padded: a column's lanes store to 16 banks, not to one
+    __shared__ __align__(16) __bf16 at[64 * RP];   // A^T chunk [k][row]
+    __shared__ __align__(16) __bf16 dt[N * RP];    // dY^T chunk [n][row]
     const int rb0 = blockIdx.x * RB;
     for (int i = threadIdx.x; i < RB * K; i += blockDim.x) {
         const int r = i / K, k = i % K, row = rb0 + r;
-        at[k * RB + r] = (__bf16)(row < M ? A[(size_t)row * lda + k] : 0.f);
+        at[k * RP + r] = (__bf16)(row < M ? A[(size_t)row * lda + k] : 0.f);
     }
     for (int i = threadIdx.x; i < RB * N; i += blockDim.x) {
         const int r = i / N, c = i % N, row = rb0 + r;
-        dt[c * RB + r] = (__bf16)(row < M ? dY[(size_t)row * ldy + c] : 0.f);
+        dt[c * RP + r] = (__bf16)(row < M ? dY[(size_t)row * ldy + c] : 0.f);
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -420,8 +423,8 @@ __global__ void __launch_bounds__(256) k_gemm_wgrad(int M, int K, const float *_
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int r0 = 0; r0 < RB; r0 += 32) {
             const int rq = r0 + (lane >> 4) * 8;
-            const bf16x8 a = *(const bf16x8 *)(at + (tk * 16 + (lane & 15)) * RB + rq);
-            const bf16x8 b = *(const bf16x8 *)(dt + (tn * 16 + (lane & 15)) * RB + rq);
+            const bf16x8 a = *(const bf16x8 *)(at + (tk * 16 + (lane & 15)) * RP + rq);
+            const bf16x8 b = *(const bf16x8 *)(dt + (tn * 16 + (lane & 15)) * RP + rq);
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
         }
         const int col = tn * 16 + (lane & 15);
@@ -435,28 +438,63 @@ __global__ void __launch_bounds__(256) k_gemm_wgrad(int M, int K, const float *_
 }
 
 // out[e] += sum over blocks b (in order) of part[b][e], e < m.
-__global__ void k_sum_parts(int nblocks, int m, const float *__restrict__ part, float *__restrict__ out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= m) return;
-    float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += part[(size_t)b * m + e];
-    out[e] += s;
+//
+// One chain of additions for each entry, as long as there are blocks: what
+// bounds it is how fast the chain is fed.  A thread that loaded its own terms
+// waited for memory at each (470 us for 2,076 partial 64 x 64 matrices, 34 MB);
+// here sixteen wavefronts bring 64 blocks' terms of 64 entries to LDS while the
+// first adds the 64 before them (24 us).
+constexpr int SUM_ROWS = 64;
+__global__ void __launch_bounds__(1024) k_sum_parts(int nblocks, int m, const float *__restrict__ part,
+                                                    float *__restrict__ out) {
+    __shared__ float sl[2][SUM_ROWS][64];
+    const int c = threadIdx.x & 63, q = threadIdx.x >> 6, e = blockIdx.x * 64 + c;
+    constexpr int U = SUM_ROWS / 16;
+    float s = 0.f, v[U];
+    auto fetch = [&](int b0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int b = b0 + q + 16 * u;
+            v[u] = (b < nblocks && e < m) ? part[(size_t)b * m + e] : 0.f;
+        }
+    };
+    fetch(0);
+    for (int b0 = 0, turn = 0; b0 < nblocks; b0 += SUM_ROWS, turn ^= 1) {
+#pragma unroll
+        for (int u = 0; u < U; u++) sl[turn][q + 16 * u][c] = v[u];
+        __syncthreads();
+        fetch(b0 + SUM_ROWS);
+        if (q == 0) {
+            const int rows = min(SUM_ROWS, nblocks - b0);
+            if (rows == SUM_ROWS) {
+#pragma unroll
+                for (int r = 0; r < SUM_ROWS; r++) s += sl[turn][r][c];
+            } else {
+                for (int r = 0; r < rows; r++) s += sl[turn][r][c];
+            }
+        }
+    }
+    if (q == 0 && e < m) out[e] += s;
 }
 
 // part[block][c] = sum of dY[r][c] over the rows r = block, block + grid,
-// ... (one thread per column; k_sum_parts finishes the sum).
+// ... (one thread per column; k_sum_parts finishes the sum).  32 rows are asked
+// for at a time and added in order: 130 -> 13 us at 132,864 rows.
 __global__ void k_colsum(int M, int N, const float *__restrict__ dY, int ldy, float *__restrict__ part) {
+    constexpr int U = 32;
     const int c = threadIdx.x;
     if (c >= N) return;
     float s = 0.f;
-    for (int r = blockIdx.x; r < M; r += gridDim.x) s += dY[(size_t)r * ldy + c];
+    long long r = blockIdx.x;
+    for (; r + (U - 1) * (long long)gridDim.x < M; r += U * (long long)gridDim.x) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = dY[(size_t)(r + u * (long long)gridDim.x) * ldy + c];
+#pragma unroll
+        for (int u = 0; u < U; u++) s += v[u];
+    }
+    for (; r < M; r += gridDim.x) s += dY[(size_t)r * ldy + c];
     part[(size_t)blockIdx.x * N + c] = s;
-}
-
-// dZ = dY * hs'(Z)
-__global__ void k_act_bwd(size_t m, const float *__restrict__ dY, const float *__restrict__ Z, float *__restrict__ dZ) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i < m) dZ[i] = dY[i] * hsw_grad(Z[i]);
 }
 
 // Materialise the edges of the selected particles: X [E][32], Bv [E][16]
@@ -564,21 +602,26 @@ __global__ void __launch_bounds__(256) k_ecn_head_fwd(int E, const float *__rest
     *(float4 *)(O + (size_t)e * 4) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
-// Head backward, one thread per edge: dO_k = u (B_k . D[pe]); db3 and
-// dW3 [64][4] += H2^T dO (block partial sums in LDS, then atomics); and
+// Head backward: dO_k = u (B_k . D[pe]); db3 and
+// dW3 [64][4] += H2^T dO; and
 // dZ2 = (dO W3^T) hs'(Z2) [E][64] for the hidden layers.
 // Per block, into part[block][HEAD_PARTS]: dW3 [64][4], db3 [4], dL [16][4]
-// (k_sum_parts adds the blocks in order).
+// (k_sum_parts adds the blocks in order).  Bound by H2, Z2 and dZ2: a row per
+// thread, and sums that read H2 16 floats at a time, took 187 us for 132,864
+// edges, whole rows through LDS 30 us.
 constexpr int HEAD_PARTS = Mpn::HID * Mpn::NOUT + Mpn::NOUT + Mpn::NF * Mpn::NOUT;
 __global__ void __launch_bounds__(256) k_ecn_head_bwd(int E, const int *__restrict__ pe, const float *__restrict__ Bv,
                                                       const float *__restrict__ D, const float *__restrict__ H2,
                                                       const float *__restrict__ Z2, const float *__restrict__ X,
                                                       const float *__restrict__ W3, float *__restrict__ dZ2,
                                                       float *__restrict__ part) {
+    constexpr int TR = 64;                          // edges whose rows are in LDS at a time
     __shared__ float sdo[256][4];
     __shared__ __align__(16) float w3[Mpn::HID * Mpn::NOUT];
-    for (int q = threadIdx.x; q < Mpn::HID * Mpn::NOUT; q += blockDim.x) w3[q] = W3[q];
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float sh[TR][Mpn::HID], sx[TR][Mpn::NF];
+    const int t = threadIdx.x;
+    for (int q = t; q < Mpn::HID * Mpn::NOUT; q += blockDim.x) w3[q] = W3[q];
+    const int eb = blockIdx.x * blockDim.x, e = eb + t;
     float d[4] = {0.f, 0.f, 0.f, 0.f};
     if (e < E) {
         const float *b = Bv + (size_t)e * 16;
@@ -587,34 +630,43 @@ __global__ void __launch_bounds__(256) k_ecn_head_bwd(int E, const int *__restri
         for (int k = 0; k < 4; k++) d[k] = b[12] * (b[3 * k] * dm[0] + b[3 * k + 1] * dm[1] + b[3 * k + 2] * dm[2]);
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++) sdo[threadIdx.x][k] = d[k];
+    for (int k = 0; k < 4; k++) sdo[t][k] = d[k];
     __syncthreads();
-    if (e < E) {
-        const float *z = Z2 + (size_t)e * Mpn::HID;
-        float *dz = dZ2 + (size_t)e * Mpn::HID;
-        for (int h = 0; h < Mpn::HID; h++) {
-            const float4 wr = ((const float4 *)w3)[h];
-            dz[h] = (d[0] * wr.x + d[1] * wr.y + d[2] * wr.z + d[3] * wr.w) * hsw_grad(z[h]);
-        }
-    }
-    // thread t: dW3[t / 4][t % 4] over the block's edges, in edge order
-    const int hrow = threadIdx.x >> 2, kk = threadIdx.x & 3;
-    const int eb = blockIdx.x * blockDim.x;
-    float *pb = part + (size_t)blockIdx.x * HEAD_PARTS;
-    float s = 0.f;
-    for (int q = 0; q < 256 && eb + q < E; q++) s += H2[(size_t)(eb + q) * 64 + hrow] * sdo[q][kk];
-    pb[hrow * 4 + kk] = s;
+    // thread t: dW3[t / 4][t % 4] over the block's edges, in edge order;
     // threads 0..63: dL[t / 4][t % 4]; threads 64..67: db3
-    if (threadIdx.x < Mpn::NF * Mpn::NOUT) {
-        float sl = 0.f;
-        for (int q = 0; q < 256 && eb + q < E; q++) sl += X[(size_t)(eb + q) * Mpn::KIN + hrow] * sdo[q][kk];
-        pb[Mpn::HID * Mpn::NOUT + Mpn::NOUT + hrow * 4 + kk] = sl;
-    } else if (threadIdx.x < Mpn::NF * Mpn::NOUT + Mpn::NOUT) {
-        const int k = threadIdx.x - Mpn::NF * Mpn::NOUT;
-        float sb = 0.f;
-        for (int q = 0; q < 256 && eb + q < E; q++) sb += sdo[q][k];
-        pb[Mpn::HID * Mpn::NOUT + k] = sb;
+    const int hrow = t >> 2, kk = t & 3, h = t & 63, f = t & 15;
+    const float4 wr = ((const float4 *)w3)[h];
+    const int rows = min(256, E - eb);
+    float s = 0.f, sl = 0.f;
+    for (int q0 = 0; q0 < rows; q0 += TR) {
+        const int nr = min(TR, rows - q0);
+        // a thread has one column of every fourth row, so that the rows are
+        // read and written whole
+#pragma unroll 4
+        for (int r = t >> 6; r < nr; r += 4) {
+            const size_t at = (size_t)(eb + q0 + r) * Mpn::HID + h;
+            const float *o = sdo[q0 + r];
+            sh[r][h] = H2[at];
+            dZ2[at] = (o[0] * wr.x + o[1] * wr.y + o[2] * wr.z + o[3] * wr.w) * hsw_grad(Z2[at]);
+        }
+#pragma unroll
+        for (int r = t >> 4; r < nr; r += 16) sx[r][f] = X[(size_t)(eb + q0 + r) * Mpn::KIN + f];
+        __syncthreads();
+#pragma unroll 8
+        for (int r = 0; r < nr; r++) s += sh[r][hrow] * sdo[q0 + r][kk];
+        if (t < Mpn::NF * Mpn::NOUT) {
+#pragma unroll 8
+            for (int r = 0; r < nr; r++) sl += sx[r][hrow] * sdo[q0 + r][kk];
+        } else if (t < Mpn::NF * Mpn::NOUT + Mpn::NOUT) {
+#pragma unroll 8
+            for (int r = 0; r < nr; r++) sl += sdo[q0 + r][kk];
+        }
+        __syncthreads();
     }
+    float *pb = part + (size_t)blockIdx.x * HEAD_PARTS;
+    pb[hrow * 4 + kk] = s;
+    if (t < Mpn::NF * Mpn::NOUT) pb[Mpn::HID * Mpn::NOUT + Mpn::NOUT + hrow * 4 + kk] = sl;
+    else if (t < Mpn::NF * Mpn::NOUT + Mpn::NOUT) pb[Mpn::HID * Mpn::NOUT + kk] = sl;
 }
 
 // Adam (Kingma & Ba) on the FP32 master weights.
@@ -684,13 +736,16 @@ void ecn_infer(hipStream_t s, const EcnGraph &g, const EcnScales &sc, const __bf
                        n_capped);
 }
 void ecn_gemm(hipStream_t s, int M, int K, const float *A, int lda, const __bf16 *Wt, int N, const float *bias, int act,
-              float *Z, float *Y, int ldy) {
+              float *Z, float *Y, int ldy, const float *Zin) {
     const unsigned g = blocks(M, 64);
     switch (N) {
-    case 16: hipLaunchKernelGGL(k_gemm<16>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy); break;
-    case 32: hipLaunchKernelGGL(k_gemm<32>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy); break;
-    default: hipLaunchKernelGGL(k_gemm<64>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy); break;
+    case 16: hipLaunchKernelGGL(k_gemm<16>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy, Zin); break;
+    case 32: hipLaunchKernelGGL(k_gemm<32>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy, Zin); break;
+    default: hipLaunchKernelGGL(k_gemm<64>, dim3(g), dim3(256), 0, s, M, K, A, lda, Wt, bias, act, Z, Y, ldy, Zin); break;
     }
+}
+static void sum_parts(hipStream_t s, int nb, int m, const float *part, float *out) {
+    hipLaunchKernelGGL(k_sum_parts, dim3(blocks(m, 64)), dim3(1024), 0, s, nb, m, part, out);
 }
 size_t ecn_wgrad_parts(int M, int K, int N) { return (size_t)blocks(M, 64) * K * N; }
 void ecn_wgrad(hipStream_t s, int M, int K, const float *A, int lda, const float *dY, int ldy, int N, float *dW,
@@ -701,14 +756,11 @@ void ecn_wgrad(hipStream_t s, int M, int K, const float *A, int lda, const float
     case 32: hipLaunchKernelGGL(k_gemm_wgrad<32>, dim3(g), dim3(256), 0, s, M, K, A, lda, dY, ldy, part); break;
     default: hipLaunchKernelGGL(k_gemm_wgrad<64>, dim3(g), dim3(256), 0, s, M, K, A, lda, dY, ldy, part); break;
     }
-    hipLaunchKernelGGL(k_sum_parts, dim3(blocks((size_t)K * N, 256)), dim3(256), 0, s, (int)g, K * N, part, dW);
+    sum_parts(s, (int)g, K * N, part, dW);
 }
 void ecn_colsum(hipStream_t s, int M, int N, const float *dY, int ldy, float *db, float *part) {
     hipLaunchKernelGGL(k_colsum, dim3(256), dim3(64), 0, s, M, N, dY, ldy, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(64), 0, s, 256, N, part, db);
-}
-void ecn_act_bwd(hipStream_t s, size_t m, const float *dY, const float *Z, float *dZ) {
-    hipLaunchKernelGGL(k_act_bwd, dim3(blocks(m, 256)), dim3(256), 0, s, m, dY, Z, dZ);
+    sum_parts(s, 256, N, part, db);
 }
 void ecn_edges(hipStream_t s, const EcnGraph &g, const EcnScales &sc, int np, const int *sel, const int *rowp,
                float *X, float *Bv, int *pe) {
@@ -729,7 +781,7 @@ void ecn_head_bwd(hipStream_t s, int E, const int *pe, const float *Bv, const fl
                   const float *Z2, const float *X, const float *W3, float *dZ2, float *g_head, float *part) {
     const unsigned nb = blocks(E, 256);
     hipLaunchKernelGGL(k_ecn_head_bwd, dim3(nb), dim3(256), 0, s, E, pe, Bv, D, H2, Z2, X, W3, dZ2, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(blocks(HEAD_PARTS, 256)), dim3(256), 0, s, (int)nb, HEAD_PARTS, part, g_head);
+    sum_parts(s, (int)nb, HEAD_PARTS, part, g_head);
 }
 void ecn_adam(hipStream_t s, int m, float *w, const float *g, float *mo, float *ve, float lr, int t) {
     const float b1 = 0.9f, b2 = 0.999f;

@@ -100,7 +100,7 @@ class Mpn {
 void ecn_infer(hipStream_t s, const EcnGraph &g, const EcnScales &sc, const __bf16 *wb, const float *w,
                const double *gr, double *F, double cap = 0.0, unsigned long long *n_capped = nullptr);
 void ecn_gemm(hipStream_t s, int M, int K, const float *A, int lda, const __bf16 *Wt, int N, const float *bias, int act,
-              float *Z, float *Y, int ldy);
+              float *Z, float *Y, int ldy, const float *Zin = nullptr);
 // weight gradients are summed without atomics: per-block partials in
 // `part` (ecn_wgrad_parts / 256 N / ecn_head_parts floats), then added in
 // block order, so training is reproducible run to run
@@ -108,7 +108,6 @@ size_t ecn_wgrad_parts(int M, int K, int N);
 void ecn_wgrad(hipStream_t s, int M, int K, const float *A, int lda, const float *dY, int ldy, int N, float *dW,
                float *part);
 void ecn_colsum(hipStream_t s, int M, int N, const float *dY, int ldy, float *db, float *part);
-void ecn_act_bwd(hipStream_t s, size_t m, const float *dY, const float *Z, float *dZ);
 void ecn_edges(hipStream_t s, const EcnGraph &g, const EcnScales &sc, int np, const int *sel, const int *rowp,
                float *X, float *Bv, int *pe);
 void ecn_target(hipStream_t s, int n, int np, const int *sel, const double *F, const double *g, float acc, float *y);

@@ -139,11 +139,10 @@ void Mpn::backward(const EcnSample &s) {
     ecn_head_bwd(st, E, s.pe, s.Bv, D_, H2_, Z2_, s.X, w + OFF_W3, dZ_, g + OFF_W3, part_);
     ecn_wgrad(st, E, HID, H1_, HID, dZ_, HID, HID, g + OFF_W2, part_);
     ecn_colsum(st, E, HID, dZ_, HID, g + OFF_B2, part_);
-    // dH1 = dZ2 W2^T, dZ1 = dH1 hs'(Z1)
-    ecn_gemm(st, E, HID, dZ_, HID, wb + B_W2, HID, nullptr, 0, nullptr, dH_, HID);
-    ecn_act_bwd(st, (size_t)E * HID, dH_, Z1_, dZ_);
-    ecn_wgrad(st, E, KIN, s.X, KIN, dZ_, HID, HID, g + OFF_W1, part_);
-    ecn_colsum(st, E, HID, dZ_, HID, g + OFF_B1, part_);
+    // dZ1 = (dZ2 W2^T) hs'(Z1)
+    ecn_gemm(st, E, HID, dZ_, HID, wb + B_W2, HID, nullptr, 0, nullptr, dH_, HID, Z1_);
+    ecn_wgrad(st, E, KIN, s.X, KIN, dH_, HID, HID, g + OFF_W1, part_);
+    ecn_colsum(st, E, HID, dH_, HID, g + OFF_B1, part_);
 }
 
 void Mpn::train_steps(int iters, float lr, uint64_t seed) {
