@@ -190,6 +190,7 @@ struct ssasdpd_engine {
     EdgeRec *erow_alt = nullptr;
     // binning / tree
     double *xtree = nullptr, *spts = nullptr, *d_bbox = nullptr;
+    float4 *near = nullptr;
     PRec *rec = nullptr;        // packed gather records, written by the predictor
     bool any_solid = true;      // some particle is fixed (solidTag, static)
     bool rec_ready = false;     // rec holds this step's post-predictor state
@@ -354,7 +355,7 @@ struct ssasdpd_engine {
         ps = nullptr;
         ring.release();
         dfree(init);
-        dfree(xtree); dfree(spts); dfree(d_bbox); dfree(d_bbtmp); dfree(rec);
+        dfree(xtree); dfree(spts); dfree(near); dfree(d_bbox); dfree(d_bbtmp); dfree(rec);
         if (h_bbox) (void)hipHostFree(h_bbox);
         h_bbox = nullptr;
         dfree(sorted); dfree(cell_of); dfree(cell_count); dfree(cell_start); dfree(cell_fill);
@@ -545,6 +546,7 @@ struct ssasdpd_engine {
         x = dalloc<double>(n3); v = dalloc<double>(n3); vt = dalloc<double>(n3); F = dalloc<double>(n3);
         Fbp = dalloc<double>(n3); normal = dalloc<double>(n3); xtree = dalloc<double>(n3);
         spts = dalloc<double>(4 * (size_t)n);
+        near = dalloc<float4>(n);
         rec = dalloc<PRec>(n);
         rho = dalloc<double>(n); old_rho = dalloc<double>(n); Frho = dalloc<double>(n); mass = dalloc<double>(n);
         nu = dalloc<double>(n); bvf = dalloc<double>(n);
@@ -920,7 +922,7 @@ qwork = dalloc<char>(q_work_bytes(n));
             cell_fill = dalloc<int>(cell_cap);
         }
         bin_points(st, xtree, n, dim, grid, cell_of, cell_count, cell_start, cell_fill, sorted, spts, scan_tmp,
-                   &derr->crowded);
+                   &derr->crowded, near);
         bool want_kd = static_domain || (flags & SSASDPD_FLAG_ANN_ORDER_MOVING);
         if (want_kd && !(static_domain && kd_built)) {
             kd_build(st, xtree, n, dim, kd, kd_work, kd_work_sz);
@@ -952,7 +954,7 @@ qwork = dalloc<char>(q_work_bytes(n));
             const FinishArgs fa{nr, fin_diag ? nullptr : Dij, fin_diag ? nullptr : ntype, erow, mass, rho, type,
                                 rec_ready ? rec : nullptr, fin_diag ? Ddiag : nullptr, Dmat, S, T};
             // LDS list slots sized by the previous search's longest list
-            fr_search(st, x, n, spts, sorted, cell_start, n, dim, h, grid, kd.valid ? &kd : nullptr, W, nidx, nr2,
+            fr_search(st, x, n, spts, near, cell_start, n, dim, h, grid, kd.valid ? &kd : nullptr, W, nidx, nr2,
                       deg, derr, nullptr, &fa, last_max_deg);
             ph_end(1);
             // the host waits for the search's overflow flag only, not for
@@ -2638,6 +2640,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
     Arena a;
     double *stage = nullptr, *dp, *dq, *sp, *bb;
     unsigned long long *bbt;
+    float4 *near;
     int *srt, *cof, *dg, *row32;
     int64_t *row64;
     DevErr *de;
@@ -2646,6 +2649,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
         dp = r.take<double>(3 * (size_t)n);
         dq = r.take<double>(3 * (size_t)mq);
         sp = r.take<double>(4 * (size_t)n);
+        near = r.take<float4>(n);
         bb = r.take<double>(8);
         bbt = r.take<unsigned long long>(8);
         srt = r.take<int>(n);
@@ -2676,7 +2680,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
         cf = r.take<int>(g.ncell + 1);
         stmp = r.take<char>(std::max(scan_tmp_bytes(g.ncell + 8), scan_tmp_bytes((size_t)std::max(n, mq) + 8)));
     });
-    bin_points(st, dp, n, dim, g, cof, cc, cs, cf, srt, sp, stmp);
+    bin_points(st, dp, n, dim, g, cof, cc, cs, cf, srt, sp, stmp, nullptr, near);
     KdDev kd;
     Arena k;
     // (the tree decides the order of a list, not its length; its build also
@@ -2721,7 +2725,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
             ci = r.take<int>(tot);
             cr = r.take<double>(tot);
         });
-        fr_search(st, dq, m, sp, srt, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr, nullptr, W);
+        fr_search(st, dq, m, sp, near, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr, nullptr, W);
         csr_lists(st, m, W, dg, row32, oi, orr, ci, cr);
         d2h(st, idx, ci, tot);
         if (r2) d2h(st, r2, cr, tot);

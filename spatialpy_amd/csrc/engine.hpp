@@ -168,8 +168,9 @@ void grid_setup(const double *pts_host_bbox, int n, int dim, double h, Grid &g);
 constexpr int FR_MAX_CELL = 4096;
 void bin_points(hipStream_t s, const double *pts, int n, int dim, const Grid &g, int *cell_of,
                 int *cell_count, int *cell_start, int *cell_fill, int *sorted, double *spts,
-                void *scan_tmp,    // spts: sorted points [n][4] (x, y, z, 0)
-                int *crowded = nullptr);   // raised to a cell's count past FR_MAX_CELL
+                void *scan_tmp,    // spts: sorted points [n][4] (x, y, z, index as an integer)
+                int *crowded = nullptr,    // raised to a cell's count past FR_MAX_CELL
+                float4 *near = nullptr);   // the sorted points in single precision, for the search's first pass
 // Within each cell of a binning, the point indices of sorted[] in ascending
 // order (the scatter's atomics leave them in arrival order).  spts is not
 // reordered: the result is an ordering, not a binning to search.
@@ -207,8 +208,8 @@ struct FinishArgs {
     const double *Dmat;
     int S, T;
 };
-void fr_search(hipStream_t s, const double *q, int m, const double *spts, const int *sorted,
-               const int *cell_start, int n, int dim, double h, const Grid &g, const KdDev *kd,
+void fr_search(hipStream_t s, const double *q, int m, const double *spts, const float4 *near, const int *cell_start,
+               int n, int dim, double h, const Grid &g, const KdDev *kd,
                int W, int *out_idx, double *out_r2, int *deg, DevErr *err, const int *query_order,
                const FinishArgs *fin = nullptr, int slots_hint = 0);
 // the lists' lengths alone (deg, and the longest in err->max_deg)

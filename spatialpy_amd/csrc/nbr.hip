@@ -230,6 +230,16 @@ __device__ __forceinline__ int cell_key(const int c[3], const Grid &g) {
     return t * (g.tile[0] * g.tile[1] * g.tile[2]) + w;
 }
 
+// A position in units of the cells' side from the grid's corner, in single
+// precision (see near_limit).
+__device__ __forceinline__ float4 in_cells(const double x[3], int dim, const Grid &g) {
+    float u[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        if (d < dim) u[d] = (float)((x[d] - g.origin[d]) * g.inv_cell);
+    return make_float4(u[0], u[1], u[2], 0.f);
+}
+
 // crowded: raised to a cell's count when it passes FR_MAX_CELL
 __global__ void k_cell_count(const double *pts, int n, int dim, Grid g, int *cell_of, int *count, int *crowded) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -245,28 +255,32 @@ __global__ void k_cell_count(const double *pts, int n, int dim, Grid g, int *cel
     if (crowded && k > FR_MAX_CELL) atomicMax(crowded, k);
 }
 
-__global__ void k_cell_scatter(const double *pts, int n, int dim, const int *cell_of, const int *start,
-                               int *fill, int *sorted, double *spts) {
+__global__ void k_cell_scatter(const double *pts, int n, int dim, Grid g, const int *cell_of, const int *start,
+                               int *fill, int *sorted, double *spts, float4 *near) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int c = cell_of[i];
     int p = start[c] + atomicAdd(&fill[c], 1);
     sorted[p] = i;
-    // one 32-byte record per point: a candidate is two 16-byte loads
+    // one 32-byte record per point (x, y, z, its index): a candidate is two
+    // 16-byte loads
+    double x[3] = {0.0, 0.0, 0.0};
+    for (int d = 0; d < dim; d++) x[d] = pts[(size_t)d * n + i];
     double2 *o = (double2 *)(spts + 4 * (size_t)p);
-    o[0] = make_double2(pts[i], dim > 1 ? pts[(size_t)n + i] : 0.0);
-    o[1] = make_double2(dim > 2 ? pts[2 * (size_t)n + i] : 0.0, 0.0);
+    o[0] = make_double2(x[0], x[1]);
+    o[1] = make_double2(x[2], __longlong_as_double(i));
+    if (near) near[p] = in_cells(x, dim, g);
 }
 
 void bin_points(hipStream_t s, const double *pts, int n, int dim, const Grid &g, int *cell_of, int *cell_count,
-                int *cell_start, int *cell_fill, int *sorted, double *spts, void *scan_tmp, int *crowded) {
+                int *cell_start, int *cell_fill, int *sorted, double *spts, void *scan_tmp, int *crowded, float4 *near) {
     HIP_OK(hipMemsetAsync(cell_count, 0, sizeof(int) * g.ncell, s));
     HIP_OK(hipMemsetAsync(cell_fill, 0, sizeof(int) * g.ncell, s));
     hipLaunchKernelGGL(k_cell_count, dim3((n + 255) / 256), dim3(256), 0, s, pts, n, dim, g, cell_of, cell_count,
                        crowded);
     exclusive_scan_i32(s, cell_count, cell_start, g.ncell, scan_tmp);
-    hipLaunchKernelGGL(k_cell_scatter, dim3((n + 255) / 256), dim3(256), 0, s, pts, n, dim, cell_of, cell_start,
-                       cell_fill, sorted, spts);
+    hipLaunchKernelGGL(k_cell_scatter, dim3((n + 255) / 256), dim3(256), 0, s, pts, n, dim, g, cell_of, cell_start,
+                       cell_fill, sorted, spts, near);
 }
 
 // One thread per cell: insertion sort of the cell's indices (cells hold a
@@ -893,10 +907,22 @@ __device__ __forceinline__ double edge_dij(double mi, double ri, double mj, doub
 }
 
 // SLOTS 0: the lists' lengths only.
-template <int SLOTS>
+// NEAR: of the candidates in a query's 27 cells (57 for 9 neighbours) most are
+// told apart by their single-precision positions in units of a cell (near,
+// 16 bytes each), with room for those positions' rounding (see near_limit);
+// only what remains is loaded and compared in double precision.  What bounds
+// the search is the address unit and L1 (a wavefront's 64 queries load from 64
+// different lines at each candidate, three loads each before: 212 million
+// accesses for a million queries, 136 now); a query with more than SLOTS such
+// candidates takes the plain way.  Cylinder: 0.62 -> 0.56 ms at 1,000,000
+// particles, 70 -> 63 us at 64,000 (the binning, which writes near, +11 us at a
+// million).  Also tried: rows of cells staged in LDS (0.68 ms: queries go in the
+// particles' order, in which few runs of cells join up), and the event loop's
+// rows written four lanes to a row (0.56 ms: no gain).
+template <int SLOTS, bool NEAR>
 __global__ void __launch_bounds__(WAVE)
-k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts, const int *__restrict__ sorted,
-            const int *__restrict__ cell_start, int n, int dim, double h, Grid g, KdView kd, int W,
+k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts, const float4 *__restrict__ near,
+            float lim_near, const int *__restrict__ cell_start, int n, int dim, double h, Grid g, KdView kd, int W,
             int *__restrict__ out_idx, double *__restrict__ out_r2, int *__restrict__ deg, DevErr *err,
             const int *__restrict__ order, FinishArgs fin, int has_fin) {
     __shared__ int l_idx[SLOTS > 0 ? SLOTS * WAVE : 1];
@@ -938,7 +964,11 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
                 hi[d] = min(c + 1, g.dims[d] - 1);
             }
         }
-        const double sq = h * h;
+        // a point at squared distance d belongs to the list if d <= h * h, d != 0
+        // and sqrt(d) <= h; the root is monotone, so that is one comparison
+        // with the largest such d
+        double lim = h * h;
+        while (sqrt(lim) > h) lim = __longlong_as_double(__double_as_longlong(lim) - 1);
         // the candidate rows' bounds, all loaded before the first is used
         int rb[9], re[9], nrow = 0;
         for (int cz = lo[2]; cz <= hi[2]; cz++)
@@ -963,31 +993,69 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
             }
             cnt++;
         };
-        // candidates in visit order, fetched CB at a time (positions and
-        // tree indices together) so one round trip serves CB of them
-        constexpr int CB = 4;
-        for (int r = 0; r < nrow; r++) {
-            const int pe = re[r];
-            for (int p0 = rb[r]; p0 < pe; p0 += CB) {
-                double2 a[CB], b[CB];
-                int jj[CB];
+        auto exact = [&](const double2 &a, const double2 &b) {
+            double dist = 0.0;
+            double t0 = qp[0] - a.x;
+            dist = dist + t0 * t0;
+            if (dim > 1) { double t1 = qp[1] - a.y; dist = dist + t1 * t1; }
+            if (dim > 2) { double t2 = qp[2] - b.x; dist = dist + t2 * t2; }
+            if (dist <= lim && dist != 0.0) accept((int)__double_as_longlong(b.y), dist);
+        };
+        // candidates in visit order, fetched CB at a time so one round trip
+        // serves CB of them
+        constexpr int CB = 4, CN = 8;
+        bool plain = true;
+        if constexpr (NEAR) {
+            const float4 qn = in_cells(qp, dim, g);
+            int found = 0;
+            for (int r = 0; r < nrow; r++) {
+                const int pe = re[r];
+                for (int p0 = rb[r]; p0 < pe; p0 += CN) {
+                    float4 c[CN];
 #pragma unroll
-                for (int u = 0; u < CB; u++) {
-                    const int p = p0 + u < pe ? p0 + u : p0;
-                    const double2 *sp = (const double2 *)(spts + 4 * (size_t)p);
-                    a[u] = sp[0];
-                    b[u] = sp[1];
-                    jj[u] = SLOTS > 0 ? sorted[p] : 0;
+                    for (int u = 0; u < CN; u++) c[u] = near[p0 + u < pe ? p0 + u : p0];
+#pragma unroll
+                    for (int u = 0; u < CN; u++) {
+                        const float dx = qn.x - c[u].x, dy = qn.y - c[u].y, dz = qn.z - c[u].z;
+                        // (not a number: left to the exact test)
+                        if (p0 + u < pe && !(dx * dx + dy * dy + dz * dz > lim_near)) {
+                            if (found < SLOTS) LI(found) = p0 + u;
+                            found++;
+                        }
+                    }
                 }
+            }
+            plain = found > SLOTS;
+            if (!plain) {
+                for (int k0 = 0; k0 < found; k0 += CB) {
+                    double2 a[CB], b[CB];
 #pragma unroll
-                for (int u = 0; u < CB; u++) {
-                    if (p0 + u >= pe) break;
-                    double dist = 0.0;
-                    double t0 = qp[0] - a[u].x;
-                    dist = dist + t0 * t0;
-                    if (dim > 1) { double t1 = qp[1] - a[u].y; dist = dist + t1 * t1; }
-                    if (dim > 2) { double t2 = qp[2] - b[u].x; dist = dist + t2 * t2; }
-                    if (dist <= sq && dist != 0.0 && sqrt(dist) <= h) accept(jj[u], dist);
+                    for (int u = 0; u < CB; u++) {
+                        const double2 *sp = (const double2 *)(spts + 4 * (size_t)LI(k0 + u < found ? k0 + u : k0));
+                        a[u] = sp[0];
+                        b[u] = sp[1];
+                    }
+                    // (the list grows behind the places read)
+#pragma unroll
+                    for (int u = 0; u < CB; u++)
+                        if (k0 + u < found) exact(a[u], b[u]);
+                }
+            }
+        }
+        if (plain) {
+            for (int r = 0; r < nrow; r++) {
+                const int pe = re[r];
+                for (int p0 = rb[r]; p0 < pe; p0 += CB) {
+                    double2 a[CB], b[CB];
+#pragma unroll
+                    for (int u = 0; u < CB; u++) {
+                        const double2 *sp = (const double2 *)(spts + 4 * (size_t)(p0 + u < pe ? p0 + u : p0));
+                        a[u] = sp[0];
+                        b[u] = sp[1];
+                    }
+#pragma unroll
+                    for (int u = 0; u < CB; u++)
+                        if (p0 + u < pe) exact(a[u], b[u]);
                 }
             }
         }
@@ -1072,7 +1140,35 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
     if (tl == 0) atomicMax(&err->max_deg, mx);
 }
 
-void fr_search(hipStream_t s, const double *q, int m, const double *spts, const int *sorted, const int *cell_start,
+// The squared distance, in cells and single precision, past which a point is
+// farther than h for certain.  Of two positions at most `span` cells from the
+// corner each component is off by at most 2^-24 span, their difference by
+// 2^-23 span and one rounding, the distance by sqrt(3) times that and 1e-6 of
+// itself: 4 2^-23 span + 1e-5 covers it.  (A span past 2^20 leaves the filter
+// little to tell apart, and it lets everything through.)
+static float near_limit(const Grid &g, double h) {
+    const double span = 2.0 + std::max({g.dims[0], g.dims[1], g.dims[2]});
+    const double r = h * g.inv_cell + 1e-5 + 4.0 * 1.1920928955078125e-7 * span;
+    return (float)(r * r * 1.00001);
+}
+template <int SLOTS>
+static void launch_search(hipStream_t s, const double *q, int m, const double *spts, const float4 *near,
+                          const int *cell_start, int n, int dim, double h, const Grid &g, const KdView &v, int W,
+                          int *out_idx, double *out_r2, int *deg, DevErr *err, const int *order, const FinishArgs *fin) {
+    const FinishArgs f = fin ? *fin : FinishArgs{};
+    const dim3 grid = xcd_grid((m + WAVE - 1) / WAVE);
+    if constexpr (SLOTS > 0) {
+        if (near) {
+            hipLaunchKernelGGL((k_fr_search<SLOTS, true>), grid, dim3(WAVE), 0, s, q, m, spts, near, near_limit(g, h),
+                               cell_start, n, dim, h, g, v, W, out_idx, out_r2, deg, err, order, f, fin ? 1 : 0);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_fr_search<SLOTS, false>), grid, dim3(WAVE), 0, s, q, m, spts, nullptr, 0.f, cell_start, n,
+                       dim, h, g, v, W, out_idx, out_r2, deg, err, order, f, fin ? 1 : 0);
+}
+
+void fr_search(hipStream_t s, const double *q, int m, const double *spts, const float4 *near, const int *cell_start,
                int n, int dim, double h, const Grid &g, const KdDev *kd, int W, int *out_idx, double *out_r2,
                int *deg, DevErr *err, const int *order, const FinishArgs *fin, int slots_hint) {
     KdView v{};
@@ -1080,27 +1176,24 @@ void fr_search(hipStream_t s, const double *q, int m, const double *spts, const 
         v.parent = kd->parent; v.depth = kd->depth; v.cd = kd->cd; v.is_hi = kd->is_hi;
         v.leaf_of = kd->leaf_of; v.cv = kd->cv; v.valid = 1;
     }
-    const FinishArgs f = fin ? *fin : FinishArgs{};
-    const dim3 grid = xcd_grid((m + WAVE - 1) / WAVE);
-    const int hf = fin ? 1 : 0;
-    if (slots_hint <= FR_SLOT_CHOICES[0])
-        hipLaunchKernelGGL(k_fr_search<12>, grid, dim3(WAVE), 0, s, q, m, spts, sorted, cell_start, n, dim, h, g, v, W,
-                           out_idx, out_r2, deg, err, order, f, hf);
-    else if (slots_hint <= FR_SLOT_CHOICES[1])
-        hipLaunchKernelGGL(k_fr_search<16>, grid, dim3(WAVE), 0, s, q, m, spts, sorted, cell_start, n, dim, h, g, v, W,
-                           out_idx, out_r2, deg, err, order, f, hf);
-    else if (slots_hint <= FR_SLOT_CHOICES[2])
-        hipLaunchKernelGGL(k_fr_search<24>, grid, dim3(WAVE), 0, s, q, m, spts, sorted, cell_start, n, dim, h, g, v, W,
-                           out_idx, out_r2, deg, err, order, f, hf);
+    // (a query finds itself among the near candidates)
+    const int want = slots_hint + (near ? 1 : 0);
+    // lists past every choice: their near candidates do not fit either
+    if (want > FR_SLOT_CHOICES[3]) near = nullptr;
+    if (want <= FR_SLOT_CHOICES[0])
+        launch_search<12>(s, q, m, spts, near, cell_start, n, dim, h, g, v, W, out_idx, out_r2, deg, err, order, fin);
+    else if (want <= FR_SLOT_CHOICES[1])
+        launch_search<16>(s, q, m, spts, near, cell_start, n, dim, h, g, v, W, out_idx, out_r2, deg, err, order, fin);
+    else if (want <= FR_SLOT_CHOICES[2])
+        launch_search<24>(s, q, m, spts, near, cell_start, n, dim, h, g, v, W, out_idx, out_r2, deg, err, order, fin);
     else
-        hipLaunchKernelGGL(k_fr_search<32>, grid, dim3(WAVE), 0, s, q, m, spts, sorted, cell_start, n, dim, h, g, v, W,
-                           out_idx, out_r2, deg, err, order, f, hf);
+        launch_search<32>(s, q, m, spts, near, cell_start, n, dim, h, g, v, W, out_idx, out_r2, deg, err, order, fin);
 }
 
 void fr_count(hipStream_t s, const double *q, int m, const double *spts, const int *cell_start, int n, int dim,
               double h, const Grid &g, int *deg, DevErr *err) {
-    hipLaunchKernelGGL(k_fr_search<0>, xcd_grid((m + WAVE - 1) / WAVE), dim3(WAVE), 0, s, q, m, spts, nullptr,
-                       cell_start, n, dim, h, g, KdView{}, 0, nullptr, nullptr, deg, err, nullptr, FinishArgs{}, 0);
+    launch_search<0>(s, q, m, spts, nullptr, cell_start, n, dim, h, g, KdView{}, 0, nullptr, nullptr, deg, err,
+                     nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------

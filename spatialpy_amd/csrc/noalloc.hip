@@ -188,7 +188,7 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
     for (;;) {
         const DevErr e0{0, INT32_MAX, 0, 0, 0};
         HIP_OK(hipMemcpyAsync(de, &e0, sizeof e0, hipMemcpyHostToDevice, st));
-        if (m > 0) fr_search(st, dq, m, sp, srt, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr);
+        if (m > 0) fr_search(st, dq, m, sp, nullptr, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr);
         HIP_OK(hipMemcpyAsync(&e, de, sizeof e, hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
         if (!e.overflow) break;
