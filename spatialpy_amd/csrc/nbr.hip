@@ -914,7 +914,7 @@ __device__ __forceinline__ double edge_dij(double mi, double ri, double mj, doub
 // the search is the address unit and L1 (a wavefront's 64 queries load from 64
 // different lines at each candidate, three loads each before: 212 million
 // accesses for a million queries, 136 now); a query with more than SLOTS such
-// candidates takes the plain way.  Cylinder: 0.62 -> 0.56 ms at 1,000,000
+// candidates takes the plain way.  Cylinder: 0.62 -> 0.54 ms at 1,000,000
 // particles, 70 -> 63 us at 64,000 (the binning, which writes near, +11 us at a
 // million).  Also tried: rows of cells staged in LDS (0.68 ms: queries go in the
 // particles' order, in which few runs of cells join up), and the event loop's
@@ -1176,8 +1176,9 @@ void fr_search(hipStream_t s, const double *q, int m, const double *spts, const 
         v.parent = kd->parent; v.depth = kd->depth; v.cd = kd->cd; v.is_hi = kd->is_hi;
         v.leaf_of = kd->leaf_of; v.cv = kd->cv; v.valid = 1;
     }
-    // (a query finds itself among the near candidates)
-    const int want = slots_hint + (near ? 1 : 0);
+    // a query that is a point finds itself among the near candidates; an
+    // engine's hint is the longest list of a step before, which few reach
+    const int want = slots_hint + (near && !fin ? 1 : 0);
     // lists past every choice: their near candidates do not fit either
     if (want > FR_SLOT_CHOICES[3]) near = nullptr;
     if (want <= FR_SLOT_CHOICES[0])
