@@ -288,8 +288,8 @@ int ssasdpd_ensemble_create(const ssasdpd_desc *const *descs, int32_t n_models, 
 void ssasdpd_ensemble_destroy(ssasdpd_ensemble *m);
 /* Snapshot count K (the reference's output schedule). */
 int ssasdpd_ensemble_num_snapshots(ssasdpd_ensemble *m, int32_t *k);
-/* Event-tree width (voxels per lane under a level-1 node: 1, 2, 4, 8, 16 or
- * 32) used by every model; results do not depend on it. */
+/* Event-queue width (a node of the queue has 64 times as many voxels: 1, 2, 4,
+ * 8, 16 or 32) used by every model; results do not depend on it. */
 int ssasdpd_ensemble_set_tree_width(ssasdpd_ensemble *m, int32_t pl);
 /* Autotuner: times probe_steps steps of the ensemble (seeds as for run) at
  * widths 1, 2, 4, 8 and keeps the fastest.  ms_per_width[4] (may be NULL)

@@ -394,7 +394,7 @@ struct ssasdpd_engine {
         if (ps) erow_alt = dalloc<EdgeRec>(cap);
     }
 
-    // options set before setup (ensembles): a common event-tree width and a
+    // options set before setup (ensembles): a common node width and a
     // shared stream
     int pl_override = 0;
     hipStream_t ext_stream = nullptr;
@@ -481,9 +481,9 @@ struct ssasdpd_engine {
                   capped ? (unsigned long long *)(nn_acc + 3) : nullptr);
     }
 
-    // Level-1 nodes held in the event loop's LDS (with the levels above:
-    // about 48 KiB at the limit).  The narrowest width that fits is the
-    // fastest: each event loads one level-0 node of 64*pl firing times.
+    // Nodes whose bounds the event loop holds in LDS (8 bytes each, 32 KiB at
+    // the limit).  The narrowest width that fits is the fastest: a scan reads a
+    // node's 64*pl firing times for the voxel or two it brings.
     static constexpr int L1_MAX = 4096;
     static int auto_pl(int nv) {
         int p = 1;
@@ -493,7 +493,7 @@ struct ssasdpd_engine {
     static bool pl_valid(int p, int nv) {
         return (p == 1 || p == 2 || p == 4 || p == 8 || p == 16 || p == 32) && (nv + 64 * p - 1) / (64 * p) <= L1_MAX;
     }
-    // Level sizes/offsets for width p, tree storage and the event loop's LDS.
+    // The nodes of width p, their bounds and the event loop's LDS.
     void layout_tree(int p) {
         if (!pl_valid(p, n))
             throw HipError("too many voxels for the event tree (max 8.3M)", hipErrorUnknown, __FILE__, __LINE__);
@@ -512,7 +512,7 @@ struct ssasdpd_engine {
         while (n1 > 1) { n1 = (n1 + TREE_FAN - 1) / TREE_FAN; nodes += n1; }
         return ssa_lds_bytes(nodes, S, R, T, nnzN_, nnzG_, n_code, n_consts);
     }
-    // Change the tree width of a built queue: the levels are rebuilt from
+    // Change the node width of a built queue: the bounds are formed again from
     // the firing times, so the event sequence is unchanged.
     void set_pl(int p) {
         if (p == pl) return;
@@ -1341,7 +1341,7 @@ qwork = dalloc<char>(q_work_bytes(n));
     // ---- batched ensembles: B trajectories of the same model, seeded
     // streams, one event-loop workgroup per trajectory.  Per trajectory:
     // counts [n][S], rates [n][R], srrate / sdrate / firing times [n], the
-    // event tree and the queue scalars.
+    // nodes' bounds and the queue scalars.
     int bcap = 0;
     uint32_t *b_xx = nullptr;
     double *b_rr = nullptr, *b_sr = nullptr, *b_sd = nullptr, *b_qt = nullptr, *b_tmin = nullptr;
