@@ -2641,8 +2641,8 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
     double *stage = nullptr, *dp, *dq, *sp, *bb;
     unsigned long long *bbt;
     float4 *near;
-    int *srt, *cof, *dg, *row32;
-    int64_t *row64;
+    int *srt, *cof, *dg;
+    int64_t *row;
     DevErr *de;
     a.plan([&](Arena &r) {
         stage = r.take<double>(3 * (size_t)std::max(n, mq));
@@ -2655,8 +2655,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
         srt = r.take<int>(n);
         cof = r.take<int>(n);
         dg = r.take<int>(mq);
-        row32 = r.take<int>((size_t)mq + 1);
-        row64 = r.take<int64_t>((size_t)mq + 1);
+        row = r.take<int64_t>((size_t)mq + 1);
         de = r.take<DevErr>(1);
     });
     h2d(st, stage, pts, 3 * (size_t)n);
@@ -2678,7 +2677,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
         cc = r.take<int>(g.ncell + 1);
         cs = r.take<int>(g.ncell + 2);
         cf = r.take<int>(g.ncell + 1);
-        stmp = r.take<char>(std::max(scan_tmp_bytes(g.ncell + 8), scan_tmp_bytes((size_t)std::max(n, mq) + 8)));
+        stmp = r.take<char>(std::max(scan_tmp_bytes(g.ncell + 8), scan_tmp_bytes(mq, sizeof(int64_t))));
     });
     bin_points(st, dp, n, dim, g, cof, cc, cs, cf, srt, sp, stmp, nullptr, near);
     KdDev kd;
@@ -2705,9 +2704,8 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
     if (m > 0) {
         h2d(st, de, &e0, 1);
         fr_count(st, dq, m, sp, cs, n, dim, h, g, dg, de);
-        exclusive_scan_i32(st, dg, row32, m, stmp);
-        rows64(st, row32, m, row64);
-        d2h(st, row_ptr, row64, (size_t)m + 1);
+        exclusive_scan_i64(st, dg, row, m, stmp);
+        d2h(st, row_ptr, row, (size_t)m + 1);
         d2h(st, &e, de, 1);
         HIP_OK(hipStreamSynchronize(st));
     } else {
@@ -2726,7 +2724,7 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
             cr = r.take<double>(tot);
         });
         fr_search(st, dq, m, sp, near, cs, n, dim, h, g, &kd, W, oi, orr, dg, de, nullptr, nullptr, W);
-        csr_lists(st, m, W, dg, row32, oi, orr, ci, cr);
+        csr_lists(st, m, W, dg, row, oi, orr, ci, cr);
         d2h(st, idx, ci, tot);
         if (r2) d2h(st, r2, cr, tot);
         HIP_OK(hipStreamSynchronize(st));

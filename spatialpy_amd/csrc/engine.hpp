@@ -215,15 +215,16 @@ void fr_search(hipStream_t s, const double *q, int m, const double *spts, const 
 // the lists' lengths alone (deg, and the longest in err->max_deg)
 void fr_count(hipStream_t s, const double *q, int m, const double *spts, const int *cell_start, int n, int dim,
               double h, const Grid &g, int *deg, DevErr *err);
-// [n][3] to [3][n]; row offsets to 64 bits (m + 1 of them); lists [W][m] to rows
+// [n][3] to [3][n]; lists [W][m] to the rows that start at row[0..m-1]
 void soa3(hipStream_t s, const double *aos, int n, double *soa);
-void rows64(hipStream_t s, const int *row32, int m, int64_t *row64);
-void csr_lists(hipStream_t s, int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
-               double *cr);
+void csr_lists(hipStream_t s, int m, int W, const int *deg, const int64_t *row, const int *oi, const double *orr,
+               int *ci, double *cr);
 void kd_build(hipStream_t s, const double *pts, int n, int dim, KdDev &kd, void *work, size_t work_bytes);
 size_t kd_work_bytes(int n);
-size_t scan_tmp_bytes(long long n);
+size_t scan_tmp_bytes(long long n, size_t elem = sizeof(int));
 void exclusive_scan_i32(hipStream_t s, const int *in, int *out, long long n, void *tmp);
+// the sums in 64 bits (tmp: scan_tmp_bytes(n, sizeof(int64_t)))
+void exclusive_scan_i64(hipStream_t s, const int *in, int64_t *out, long long n, void *tmp);
 
 
 // SDPD substeps.

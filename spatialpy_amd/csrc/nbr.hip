@@ -37,46 +37,48 @@ __device__ __forceinline__ double dkey_inv(unsigned long long k) {
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive scan of int32 (3-phase: block reduce, scan of block sums, add).
+// Exclusive scan of int32 counts (3-phase: block reduce, scan of block sums,
+// add) into T: int where the total has a known bound, int64_t for the rows of
+// the stand-alone search, whose lists together may pass 2^31 entries.
 constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 4;
 constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
-__device__ int block_exclusive_scan(int v, int *lds, int &total) {
+template <class T> __device__ T block_exclusive_scan(T v, T *lds, T &total) {
     // v: thread partial; returns exclusive prefix within the block
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-    int x = v;
+    T x = v;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
-        int y = __shfl_up(x, o, WAVE);
+        T y = __shfl_up(x, o, WAVE);
         if (lane >= o) x += y;
     }
     if (lane == WAVE - 1) lds[w] = x;
     __syncthreads();
     if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int i = 0; i < SCAN_BLOCK / WAVE; i++) { int t = lds[i]; lds[i] = acc; acc += t; }
+        T acc = 0;
+        for (int i = 0; i < SCAN_BLOCK / WAVE; i++) { T t = lds[i]; lds[i] = acc; acc += t; }
         lds[SCAN_BLOCK / WAVE] = acc;
     }
     __syncthreads();
     total = lds[SCAN_BLOCK / WAVE];
-    int r = x - v + lds[w];
+    T r = x - v + lds[w];
     __syncthreads();
     return r;
 }
 
-__global__ void k_scan_tiles(const int *in, int *out, long long n, int *tile_sums) {
-    __shared__ int lds[SCAN_BLOCK / WAVE + 1];
+template <class I, class T> __global__ void k_scan_tiles(const I *in, T *out, long long n, T *tile_sums) {
+    __shared__ T lds[SCAN_BLOCK / WAVE + 1];
     long long base = (long long)blockIdx.x * SCAN_TILE + (long long)threadIdx.x * SCAN_ITEMS;
-    int v[SCAN_ITEMS];
-    int s = 0;
+    T v[SCAN_ITEMS];
+    T s = 0;
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
-        v[k] = (base + k < n) ? in[base + k] : 0;
+        v[k] = (base + k < n) ? (T)in[base + k] : (T)0;
         s += v[k];
     }
-    int total;
-    int pre = block_exclusive_scan(s, lds, total);
+    T total;
+    T pre = block_exclusive_scan(s, lds, total);
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
         if (base + k < n) out[base + k] = pre;
@@ -85,23 +87,24 @@ __global__ void k_scan_tiles(const int *in, int *out, long long n, int *tile_sum
     if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
 }
 
-__global__ void k_scan_add(int *out, long long n, const int *tile_pre) {
+template <class T> __global__ void k_scan_add(T *out, long long n, const T *tile_pre) {
     long long i = (long long)blockIdx.x * SCAN_TILE + threadIdx.x;
-    int add = tile_pre[blockIdx.x];
+    T add = tile_pre[blockIdx.x];
     for (int k = 0; k < SCAN_ITEMS; k++, i += SCAN_BLOCK)
         if (i < n) out[i] += add;
 }
 
-__global__ void k_scan_fix(const int *in, int *out, long long n) {
-    if (threadIdx.x == 0) out[n] = n > 0 ? out[n - 1] + in[n - 1] : 0;
+template <class I, class T> __global__ void k_scan_fix(const I *in, T *out, long long n) {
+    if (threadIdx.x == 0) out[n] = n > 0 ? out[n - 1] + (T)in[n - 1] : (T)0;
 }
 
-size_t scan_tmp_bytes(long long n) {
+// bytes of tmp for sums of `elem` bytes
+size_t scan_tmp_bytes(long long n, size_t elem) {
     size_t b = 0;
     long long m = n + 1;
     for (;;) {
         long long tiles = (m + SCAN_TILE - 1) / SCAN_TILE;
-        b += (size_t)(2 * tiles + 4) * sizeof(int);
+        b += (size_t)(2 * tiles + 4) * elem;
         if (tiles <= 1) break;
         m = tiles + 1;
     }
@@ -109,21 +112,27 @@ size_t scan_tmp_bytes(long long n) {
 }
 
 // out[i] = sum(in[0..i-1]); out must have n+1 entries (out[n] = total).
-void exclusive_scan_i32(hipStream_t s, const int *in, int *out, long long n, void *tmp) {
+template <class I, class T> static void exclusive_scan(hipStream_t s, const I *in, T *out, long long n, void *tmp) {
     // scan n+1 elements where in[n] is treated as 0
     long long m = n + 1;
     long long tiles = (m + SCAN_TILE - 1) / SCAN_TILE;
-    int *sums = (int *)tmp;
-    int *pre = sums + tiles + 1;
+    T *sums = (T *)tmp;
+    T *pre = sums + tiles + 1;
     // in[n] may be out of bounds: run the tile scan on n elements and fix the
     // last entry with the tile total
-    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, s, in, out, n, sums);
+    hipLaunchKernelGGL((k_scan_tiles<I, T>), dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, s, in, out, n, sums);
     if (tiles > 1) {
-        exclusive_scan_i32(s, sums, pre, tiles, (void *)(pre + tiles + 1));
-        hipLaunchKernelGGL(k_scan_add, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, s, out, n, pre);
+        exclusive_scan<T, T>(s, sums, pre, tiles, (void *)(pre + tiles + 1));
+        hipLaunchKernelGGL(k_scan_add<T>, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, s, out, n, pre);
     }
     // out[n] = out[n-1] + in[n-1]
-    hipLaunchKernelGGL(k_scan_fix, dim3(1), dim3(1), 0, s, in, out, n);
+    hipLaunchKernelGGL((k_scan_fix<I, T>), dim3(1), dim3(1), 0, s, in, out, n);
+}
+void exclusive_scan_i32(hipStream_t s, const int *in, int *out, long long n, void *tmp) {
+    exclusive_scan<int, int>(s, in, out, n, tmp);
+}
+void exclusive_scan_i64(hipStream_t s, const int *in, int64_t *out, long long n, void *tmp) {
+    exclusive_scan<int, int64_t>(s, in, out, n, tmp);
 }
 
 // ---------------------------------------------------------------------------
@@ -1198,22 +1207,19 @@ void fr_count(hipStream_t s, const double *q, int m, const double *spts, const i
 }
 
 // ---------------------------------------------------------------------------
-// Host layouts: particle-major points to component-major, 64-bit row offsets,
-// column-major lists to rows.
+// Host layouts: particle-major points to component-major, column-major lists to
+// rows.
 __global__ void k_soa3(const double *aos, int n, double *soa) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     for (int d = 0; d < 3; d++) soa[(size_t)d * n + i] = aos[3 * (size_t)i + d];
 }
-__global__ void k_rows64(const int *row32, int m, int64_t *row64) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i <= m) row64[i] = row32[i];
-}
-__global__ void k_csr(int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
+__global__ void k_csr(int m, int W, const int *deg, const int64_t *row, const int *oi, const double *orr, int *ci,
                       double *cr) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m) return;
-    const int d = deg[i], o = row32[i];
+    const int d = deg[i];
+    const int64_t o = row[i];
     for (int k = 0; k < d && k < W; k++) {
         ci[o + k] = oi[(size_t)k * m + i];
         cr[o + k] = orr[(size_t)k * m + i];
@@ -1222,13 +1228,10 @@ __global__ void k_csr(int m, int W, const int *deg, const int *row32, const int 
 void soa3(hipStream_t s, const double *aos, int n, double *soa) {
     if (n > 0) hipLaunchKernelGGL(k_soa3, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, aos, n, soa);
 }
-void rows64(hipStream_t s, const int *row32, int m, int64_t *row64) {
-    hipLaunchKernelGGL(k_rows64, dim3((unsigned)(((size_t)m + 256) / 256)), dim3(256), 0, s, row32, m, row64);
-}
-void csr_lists(hipStream_t s, int m, int W, const int *deg, const int *row32, const int *oi, const double *orr, int *ci,
-               double *cr) {
+void csr_lists(hipStream_t s, int m, int W, const int *deg, const int64_t *row, const int *oi, const double *orr,
+               int *ci, double *cr) {
     if (m > 0)
-        hipLaunchKernelGGL(k_csr, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, m, W, deg, row32, oi, orr, ci, cr);
+        hipLaunchKernelGGL(k_csr, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, m, W, deg, row, oi, orr, ci, cr);
 }
 
 }  // namespace ssa

@@ -51,9 +51,8 @@ constexpr size_t SCAN_BYTES = 4 * (std::max<size_t>(NA_MAX_CELLS, CAP_Q) + 16) +
 constexpr size_t O_OI = O_SCAN + SCAN_BYTES;                                 // ELL [W][m]
 constexpr size_t O_OR = O_OI + al(sizeof(int) * NA_MAX_WIDTH * CAP_Q);
 constexpr size_t O_DEG = O_OR + al(sizeof(double) * NA_MAX_WIDTH * CAP_Q);
-constexpr size_t O_ROW32 = O_DEG + al(sizeof(int) * CAP_Q);
-constexpr size_t O_ROW64 = O_ROW32 + al(sizeof(int) * (CAP_Q + 1));
-constexpr size_t O_CI = O_ROW64 + al(sizeof(int64_t) * (CAP_Q + 1));         // CSR out
+constexpr size_t O_ROW = O_DEG + al(sizeof(int) * CAP_Q);
+constexpr size_t O_CI = O_ROW + al(sizeof(int64_t) * (CAP_Q + 1));           // CSR out
 constexpr size_t O_CR = O_CI + al(sizeof(int) * NA_MAX_WIDTH * CAP_Q);
 constexpr size_t O_MISC = O_CR + al(sizeof(double) * NA_MAX_WIDTH * CAP_Q);  // bbox, bbox tmp, DevErr
 constexpr size_t NA_BYTES = O_MISC + 4096;
@@ -140,7 +139,8 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
     if (n > NA_MAX_POINTS || m > NA_MAX_QUERIES)
         return report_error(SSASDPD_ERR_CAPACITY, "fr_search_noalloc: at most " + std::to_string(NA_MAX_POINTS) +
                                                    " points and " + std::to_string(NA_MAX_QUERIES) + " queries");
-    if (kd_work_bytes(NA_MAX_POINTS) > KDW_BYTES || scan_tmp_bytes(std::max<long long>(NA_MAX_CELLS, CAP_Q) + 8) > SCAN_BYTES)
+    if (kd_work_bytes(NA_MAX_POINTS) > KDW_BYTES || scan_tmp_bytes(NA_MAX_CELLS + 8) > SCAN_BYTES ||
+        scan_tmp_bytes(CAP_Q, sizeof(int64_t)) > SCAN_BYTES)
         return report_error(SSASDPD_ERR_CAPACITY, "fr_search_noalloc: scratch layout too small");
     unsigned char *base = scratch_ptr();
     hipStream_t st = 0;   // the null stream: nothing created per call
@@ -151,8 +151,7 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
     void *kw = base + O_KDW, *stmp = base + O_SCAN;
     int *oi = (int *)(base + O_OI), *dg = (int *)(base + O_DEG);
     double *orr = (double *)(base + O_OR);
-    int *row32 = (int *)(base + O_ROW32);
-    int64_t *row64 = (int64_t *)(base + O_ROW64);
+    int64_t *row = (int64_t *)(base + O_ROW);
     int *ci = (int *)(base + O_CI);
     double *cr = (double *)(base + O_CR);
     double *bb = (double *)(base + O_MISC);
@@ -202,13 +201,12 @@ extern "C" int ssasdpd_fr_search_noalloc(const double *pts, int32_t n, const dou
         row_ptr[0] = 0;
         return 0;
     }
-    exclusive_scan_i32(st, dg, row32, m, stmp);
-    rows64(st, row32, m, row64);
-    HIP_OK(hipMemcpyAsync(row_ptr, row64, sizeof(int64_t) * ((size_t)m + 1), hipMemcpyDeviceToHost, st));
+    exclusive_scan_i64(st, dg, row, m, stmp);
+    HIP_OK(hipMemcpyAsync(row_ptr, row, sizeof(int64_t) * ((size_t)m + 1), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
     if (idx) {
         const size_t tot = (size_t)row_ptr[m];
-        csr_lists(st, m, W, dg, row32, oi, orr, ci, cr);
+        csr_lists(st, m, W, dg, row, oi, orr, ci, cr);
         HIP_OK(hipMemcpyAsync(idx, ci, sizeof(int) * tot, hipMemcpyDeviceToHost, st));
         if (r2) HIP_OK(hipMemcpyAsync(r2, cr, sizeof(double) * tot, hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
