@@ -136,6 +136,9 @@ struct Grid {
     // space, partial tiles included.
     int tile[3];
     int ntile[3];
+    // some extent of the box is not finite: that dimension has one cell,
+    // however far apart its finite coordinates are
+    bool open = false;
 };
 // The tiled numbering of g's cells (see Grid).
 void grid_tile(Grid &g, int dim);

@@ -189,6 +189,8 @@ void compute_bbox(hipStream_t s, const double *pts, int n, int dim, double *d_bb
 void grid_setup(const double *bb, int n, int dim, double h, Grid &g) {
     const double limit = (double)std::max<long long>(4LL * n, 1 << 20);
     double cell = h * 1.01;
+    g.open = false;
+    for (int d = 0; d < dim && d < 3; d++) g.open = g.open || !std::isfinite(bb[2 * d + 1] - bb[2 * d]);
     for (;;) {
         double tot = 1.0, c[3] = {1.0, 1.0, 1.0};
         for (int d = 0; d < dim && d < 3; d++) {
@@ -1154,8 +1156,10 @@ k_fr_search(const double *__restrict__ q, int m, const double *__restrict__ spts
 // corner each component is off by at most 2^-24 span, their difference by
 // 2^-23 span and one rounding, the distance by sqrt(3) times that and 1e-6 of
 // itself: 4 2^-23 span + 1e-5 covers it.  (A span past 2^20 leaves the filter
-// little to tell apart, and it lets everything through.)
+// little to tell apart, and it lets everything through; so does a grid with an
+// open dimension, whose one cell says nothing about the positions in it.)
 static float near_limit(const Grid &g, double h) {
+    if (g.open) return INFINITY;
     const double span = 2.0 + std::max({g.dims[0], g.dims[1], g.dims[2]});
     const double r = h * g.inv_cell + 1e-5 + 4.0 * 1.1920928955078125e-7 * span;
     return (float)(r * r * 1.00001);
