@@ -2684,8 +2684,8 @@ int ssasdpd_fr_search(const double *pts, int32_t n, const double *q, int32_t m, 
     Arena k;
     // (the tree decides the order of a list, not its length; its build also
     // refuses points that do not compare)
-    const bool nan = std::any_of(hb, hb + 2 * dim, [](double v) { return std::isnan(v); });
-    if (idx || nan) {
+    const bool open = std::any_of(hb, hb + 2 * dim, [](double v) { return !std::isfinite(v); });
+    if (idx || open) {
         char *kw;
         const size_t kws = kd_work_bytes(n), nodes = 2 * (size_t)n + 2;
         k.plan([&](Arena &r) {

@@ -408,7 +408,14 @@ __global__ void k_kd_root(const double *bb, int n, int dim, KdWork w, KdDev kd, 
     w.s_n[0] = n;
     w.s_node[0] = 0;
     for (int d = 0; d < 3; d++) {
-        w.s_lo[(size_t)d * cap] = bb[2 * d];
+        // A box from -inf to +inf has no middle to cut at: its cut would put
+        // every point on the upper side and leave that child's lower bound NaN,
+        // after which no cell is cut there again (lengths that do not compare
+        // lose against the others).  The root starts so: its one child would
+        // only add a level above all the points.  Dimension 0 is the one that
+        // others are compared with, so there the tree is refused.
+        const bool endless = d > 0 && bb[2 * d] == -INFINITY && bb[2 * d + 1] == INFINITY;
+        w.s_lo[(size_t)d * cap] = endless ? NAN : bb[2 * d];
         w.s_hi[(size_t)d * cap] = bb[2 * d + 1];
     }
     kd.parent[0] = -1;
