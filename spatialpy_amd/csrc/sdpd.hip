@@ -245,7 +245,8 @@ __device__ __forceinline__ void to_lds16(const void *src, void *dst) {
 template <typename Real, bool MOMENTUM, bool CHEM, int NSC>
 __global__ void __launch_bounds__(256) k_forces(SdpdArgs a) {
     constexpr int NR = MOMENTUM ? 256 : 1;
-    __shared__ char s_rec[NR * sizeof(PRec)];
+    __shared__ __align__(16) char s_rec[NR * sizeof(PRec)];
+    static_assert(__alignof__(s_rec) >= 16, "to_lds16 writes and double2 reads 16 bytes at a time");
     __shared__ int s_j[NR];
     const int chunk = xcd_chunk((a.n + 255) / 256);
     if (chunk < 0) return;
