@@ -1139,21 +1139,20 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 }
                 const double vol_c = __shfl(vol, peer, WAVE), t_c = __shfl(t, peer, WAVE);
                 const int tds_c = __shfl(tds, peer, WAVE), dv_c = __shfl(dv, peer, WAVE);
-                const unsigned dep_c = (unsigned)__shfl((int)(up ? 0u : dep), peer, WAVE);
-                const bool on_c = up ? __shfl(there ? 1 : 0, peer, WAVE) != 0 : act;
                 const int at_c = up ? dv_c : sv, tp_c = up ? tds_c : tsv;
                 const double *const df_c = a.data_fn ? a.data_fn + (size_t)at_c * a.n_df : nullptr;
                 lp.stage(xc);
                 double rd = 0.0, rdd = 0.0;
                 for (int j = 0; j < R; j++) {
-                    const bool now = on_c && ((dep_c >> j) & 1u);
+                    // (only the lower half has lanes with a column: a destination
+                    // takes its source's)
+                    const bool now = act && ((dep >> j) & 1u);
                     if (!__ballot(now)) continue;
                     const double p = lp.template prop<true>(j, xc, vol_c, tp_c, t_c, df_c);
                     const double pd = __shfl(p, (lane & 31) + 32, WAVE);
-                    const bool mine = ((dep >> j) & 1u) && act && !up;
 #pragma unroll
                     for (int u = 0; u < MR; u++)
-                        if (u == j && mine) {
+                        if (u == j && now) {
                             rd += p - vx.r[u];
                             vx.r[u] = p;
                             if (there) {
