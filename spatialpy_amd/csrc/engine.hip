@@ -241,6 +241,9 @@ struct ssasdpd_engine {
     uint32_t cur = 0;
     bool lists_built = false;
     bool kd_built = false;
+    // voxels with a next event: at the start (about; 64 stands for more), and when
+    // the host last saw the queue
+    long long active0 = 0, active_seen = 0;
     bool rdme_initialized = false;
     ssasdpd_stats stats{};
     int max_deg_seen = 0;
@@ -613,6 +616,11 @@ struct ssasdpd_engine {
         h2d(st, mass, d->mass, n);
         const std::vector<double> x0 = to_soa3(d->x, n), v0 = to_soa3(d->v, n);
         if (S > 0) u0.assign(d->u0, d->u0 + (size_t)n * S);
+        for (int r = 0; r < d->n_reactions; r++)
+            if (d->reactions[r].kind == 0) active0 = n;    // fires in empty voxels
+        // (only whether they are few matters)
+        for (size_t v = 0; v < u0.size() && active0 <= 64; v += S)
+            active0 += std::any_of(u0.begin() + v, u0.begin() + v + S, [](uint32_t c) { return c > 0; });
         std::vector<double> C0((size_t)n * Sc, 0.0);
         for (size_t k = 0; k < (size_t)n * Sc; k++)
             C0[k] = d->C0 ? d->C0[k] : (S == Sc && d->u0 ? (double)d->u0[k] : 0.0);
@@ -750,6 +758,7 @@ qwork = dalloc<char>(q_work_bytes(n));
             HIP_OK(hipMemsetAsync(sdrate, 0, sizeof(double) * n, st));
             QueueState q{};
             h2d(st, qs, &q, 1);
+            active_seen = active0;
         }
         DevErr e0{0, INT32_MAX, 0, 0, 0};
         h2d(st, derr, &e0, 1);
@@ -1003,6 +1012,7 @@ qwork = dalloc<char>(q_work_bytes(n));
         a.row_w = std::max(1, std::min(W, max_deg_seen));
         a.qtime = qtime; a.tmin = tmin; a.pl = pl; a.tree_nodes = tree_nodes;
         a.lds_bytes = lds_bytes;
+        a.alone = nsm_alone(n, S, R, n_code > 0, active_seen) ? 1 : 0;
         a.qs = qs;
         a.rng_kind = rng_kind; a.seed = seed; a.stream_id = 0; a.words = d_words; a.expo = d_expo; a.n_words = n_words;
         a.textbook = (flags & SSASDPD_FLAG_TEXTBOOK_SELECTION) ? 1 : 0;
@@ -1050,6 +1060,7 @@ qwork = dalloc<char>(q_work_bytes(n));
             stats.reactions = q.reactions;
             stats.diffusions = q.diffusions;
             stats.rng_words_used = q.rng_pos;
+            if (q.initialized == 1) active_seen = (long long)q.active;
             if (q.err) {
                 char buf[96];
                 snprintf(buf, sizeof buf, "SSA failed at step %u", q.err_step);
@@ -1459,17 +1470,20 @@ qwork = dalloc<char>(q_work_bytes(n));
         d2h(st, q.data(), b_qs, B);
         HIP_OK(hipStreamSynchronize(st));
         int rc = 0;
+        long long most = 0;
         stats.reactions = stats.diffusions = stats.rng_words_used = 0;
         for (int b = 0; b < B; b++) {
             stats.reactions += q[b].reactions;
             stats.diffusions += q[b].diffusions;
             stats.rng_words_used += q[b].rng_pos;
+            if (q[b].initialized == 1) most = std::max(most, (long long)q[b].active);
             if (q[b].err && !rc) {
                 char buf[128];
                 snprintf(buf, sizeof buf, "SSA failed at step %u in trajectory %d", q[b].err ? q[b].err_step : step, b);
                 rc = set_error(q[b].err, buf);
             }
         }
+        if (most > 0) active_seen = most;
         return rc;
     }
 
@@ -1570,7 +1584,8 @@ struct ssasdpd_ensemble {
         HIP_OK(hipEventRecord(e0, st));
         bool any_prog = false;
         for (auto *e : eng) any_prog = any_prog || e->n_code > 0;
-        rdme_take_step_multi(st, d_args, (int)args.size(), max_sr, lds_max(), any_prog);
+        const bool alone = std::all_of(args.begin(), args.end(), [](const RdmeArgs &a) { return a.alone != 0; });
+        rdme_take_step_multi(st, d_args, (int)args.size(), max_sr, lds_max(), any_prog, alone);
         HIP_OK(hipEventRecord(e1, st));
         HIP_OK(hipStreamSynchronize(st));
         float ms = 0.f;

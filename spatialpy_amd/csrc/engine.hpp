@@ -288,6 +288,7 @@ struct RdmeArgs {
     int pl;
     int tree_nodes;
     size_t lds_bytes;        // dynamic LDS of the event-loop kernel
+    int alone;               // see nsm_alone
     QueueState *qs;
     // random stream
     int rng_kind;            // 0 seeded (Philox), 1 replay
@@ -340,8 +341,13 @@ void rdme_queue_build(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
 size_t q_work_bytes(int n);
 void rdme_take_step(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
 void tree_rebuild(hipStream_t s, const RdmeArgs &a, int n_traj = 1);
-// one launch over n_models argument blocks (device array), common MS/MR bucket (max over the models of max(S, R)), LDS = max over models
-void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog);
+// one launch over n_models argument blocks (device array), common MS/MR bucket
+// (max over the models of max(S, R)), LDS = max over models
+void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog,
+                          bool alone);
+// Whether the event loop of a domain with `active` voxels that have a next event
+// (about: it decides the speed only) may take events one by one.
+bool nsm_alone(int n, int S, int R, bool vm, long long active);
 void vm_eval_batch(hipStream_t s, const uint32_t *code, int start, const double *K, int x_is_double, int n_x,
                    int n_df, int m, const double *xd, const uint32_t *xu, const double *vol, const double *t,
                    const double *df, double *out);

@@ -27,6 +27,13 @@
 // a hop into the voxel itself, the end of a replay stream) are carried out
 // only as the first lane of a round.
 //
+// Where consecutive events do interfere (a few voxels, or one that holds nearly
+// all molecules) a round keeps one or two of them, and costs as much as one that
+// keeps sixty, the more the more species and reactions its lanes carry.  There
+// events go one by one instead (event_alone), a lane per species and per reaction
+// of the voxel: nsm_alone chooses the kernel that can do both, and that one goes
+// by what its last rounds kept.
+//
 // The queue.  Firing times of all voxels are in memory (qtime).  Three sets,
 // divided by two horizons, hold every voxel with a finite time once: the
 // `front`, at most 64 voxels sorted by (time, voxel), one per lane, up to the
@@ -44,7 +51,9 @@
 // against the rounds): 40^3 lattice, 200,000 molecules 3.7 -> 0.36 us; 256 of
 // those trajectories at once 14.7 -> 1.6 ns; 2D dam break 3.6 -> 0.42 us; 1M
 // cylinder, 860 events a step, 2.8 -> 0.45 us; 121 voxels 3.5 -> 1.5 us;
-// custom propensities on 144 voxels 30 -> 5.2 us.  A round takes 20,000 to
+// custom propensities on 144 voxels 30 -> 5.2 us; 4 voxels 3.6 -> 5.5 us in
+// rounds, 3.0 us one by one (16 voxels with 16 species and 16 reactions 4.3 ->
+// 16.4 and 3.7 us).  A round takes 20,000 to
 // 50,000 cycles, most of them latencies (two round trips, LDS, dependent
 // FP64 operations) of a single wavefront.
 #include <hip/hip_runtime.h>
@@ -356,6 +365,22 @@ template <int MS, int MR, bool VM> struct Loop {
             lower(v, t);
         }
         nc += (int)__popcll(h);
+    }
+
+    // A voxel out of the near list: its last entry takes the place.
+    __device__ __forceinline__ void drop_near(int v) {
+        for (int c0 = 0; c0 < nc; c0 += WAVE) {
+            const unsigned long long m = __ballot(c0 + lane < nc && L.qv[c0 + lane] == v);
+            if (!m) continue;
+            nc--;
+            if (lane == 0) {
+                const int k = c0 + (int)__builtin_ctzll(m);
+                L.qt[k] = L.qt[nc];
+                L.qv[k] = L.qv[nc];
+            }
+            sync_wave();
+            break;
+        }
     }
 
     // Scan up to GROUP listed nodes: entries past the second horizon up to
@@ -677,6 +702,234 @@ template <int MS, int MR, bool VM> struct Loop {
         }
         sync_wave();
     }
+
+    // ---- one event alone --------------------------------------------------
+    // Into the sorted front, or past its horizon.
+    __device__ __forceinline__ void insert(double t, int v) {
+        if (before(tau_t, tau_v, t, v)) {
+            put(1ULL, t, v);
+            return;
+        }
+        const int at = (int)__popcll(__ballot(lane < cnt && before(ft, fv, t, v)));
+        const double last_t = rl_d(ft, WAVE - 1);
+        const int last_v = rl_i(fv, WAVE - 1);
+        const double up_t = shift_up(t, ft);
+        const int up_v = dpp_i<0x138, 0xF>(v, fv);
+        if (lane >= at) {
+            ft = lane == at ? t : up_t;
+            fv = lane == at ? v : up_v;
+        }
+        if (cnt < WAVE) {
+            cnt++;
+            return;
+        }
+        // no lane for the last of them: the horizon moves back
+        tau_t = rl_d(ft, WAVE - 1);
+        tau_v = rl_i(fv, WAVE - 1);
+        if (at < WAVE) put(1ULL, last_t, last_v);
+        else put(1ULL, t, v);
+    }
+    // Out of the sorted front: the entry of lane `at`.
+    __device__ __forceinline__ void remove(int at) {
+        const double dn_t = dpp_d<0x130, 0xF>(INFINITY, ft);     // lane l gets lane l+1's
+        const int dn_v = dpp_i<0x130, 0xF>(INT_MAX, fv);
+        if (lane >= at) {
+            ft = dn_t;
+            fv = dn_v;
+        }
+        cnt--;
+    }
+    // What bounds it is the chain of two round trips and of the additions that
+    // keep their order (about 7,000 cycles an event; a round with nothing to
+    // share takes 17,000 with 2 species and reactions, 77,000 with 16).  The
+    // evaluations are one lane each, the source's and the destination's side by
+    // side, and the front is repaired in registers.
+    // The front's first entry alone, one lane per species and per reaction of
+    // its voxel (the upper half-wave: of a hop's destination), by the operations
+    // of a round.  False, with nothing stored: an event off the common path.
+    __device__ __forceinline__ bool event_alone(QueueState &q, int &stale) {
+        static_assert(MS <= 32 && MR <= 32, "a half-wave each");
+        if (pos + 4 > n_words) return false;
+        const int l = lane & 31;
+        const bool up = lane >= 32, sp = l < S, rc = l < R;
+        const int sv = rl_i(fv, 0);
+        const double t = rl_d(ft, 0);
+        uint32_t x = sp ? xx[(size_t)sv * S + l] : 0u;
+        const double D = sp ? a.Ddiag[(size_t)sv * S + l] : 0.0;
+        double r = rc ? rrate[(size_t)sv * R + l] : 0.0;
+        double sr = srrate[sv], sd = sdrate[sv];
+        const double vol = a.vol[sv];
+        const int tsv = a.type[sv], dg = __builtin_amdgcn_readfirstlane(a.deg[sv]);
+        const EdgeRec *const row = a.erow + (size_t)sv * W;
+        EdgeRec er = row[min(lane, W - 1)];
+        fill_pool(pos + 4);
+        sync_wave();
+
+        // ---- reaction or hop, and which
+        const double rand1 = uni(pos), totrate = sr + sd;
+        const bool react = __ballot(rand1 <= sr / totrate) != 0;
+        const bool textbook = a.textbook != 0;
+        const double rv = react ? (textbook ? rand1 * totrate : rand1 * sr)
+                                : (textbook ? rand1 * totrate - sr : rand1 * sd);
+        const int m = react ? R : S;
+        const double part = react ? r : D * x;
+        int which = 0;
+        double cum = rl_d(part, 0);
+        while (which < m && rv > cum) {
+            which++;
+            cum += rl_d(part, which & 31);
+        }
+        which = __builtin_amdgcn_readfirstlane(which);
+        if (which >= m) return false;
+
+        // ---- the hop's destination
+        int dv = sv, tds = tsv;
+        double srd = 0.0, sdd = 0.0, Ddd = 0.0, qtd = INFINITY;
+        const double Dw = rl_d(D, which & 31);
+        if (!react) {
+            const double rand2 = uni(pos + 1) * Dw;
+            int jd = -1;
+            double cum2 = 0.0;
+            for (int k0 = 0; k0 < dg && jd < 0; k0 += WAVE) {
+                if (k0 > 0) er = row[min(k0 + lane, W - 1)];
+                const double w = er.D * L.Dmat[which * T + (T > 1 && k0 + lane < dg ? er.type - 1 : 0)];
+                for (int k = 0; k < WAVE && k0 + k < dg; k++) {
+                    cum2 += rl_d(w, k);
+                    if (cum2 > rand2) {
+                        jd = rl_i(er.j, k);
+                        break;
+                    }
+                }
+            }
+            jd = __builtin_amdgcn_readfirstlane(jd);
+            if (jd < 0 || jd == sv) return false;
+            dv = jd;
+            if (up) {
+                x = sp ? xx[(size_t)dv * S + l] : 0u;
+                r = rc ? rrate[(size_t)dv * R + l] : 0.0;
+            }
+            srd = srrate[dv];
+            sdd = sdrate[dv];
+            Ddd = a.Ddiag[(size_t)dv * S + which];
+            qtd = qtime[dv];
+            tds = a.type[dv];
+        }
+
+        // ---- the event
+        const bool side = !up || !react;                     // lanes with a voxel of the event
+        const unsigned dep = (unsigned)__builtin_amdgcn_readfirstlane((int)L.dep[react ? S + which : which]);
+        const int d = react && sp && !up ? L.dN[which * MS + l] : 0;
+        unsigned long long changed = 0;
+        if (react) {
+            changed = __ballot(d != 0);
+            x += (uint32_t)d;
+            for (unsigned long long h = changed; h; h &= h - 1) {
+                const int s = (int)__builtin_ctzll(h);
+                sd += rl_d(D, s) * rl_i(d, s);
+            }
+        } else if (l == which) {
+            x += up ? 1u : ~0u;
+        }
+        const bool mine = rc && side && ((dep >> l) & 1u);
+        if (dep) {
+            const Rxn *const re = L.rx + (rc ? l : 0);
+            const int kind = re->kind, at = lane & 32;
+            const int xa = __shfl((int)x, at + (re->a & 31), WAVE), xb = __shfl((int)x, at + (re->b & 31), WAVE);
+            double p;
+            if (kind == 0) {
+                p = re->k * vol;
+            } else {
+                p = re->k * xa;
+                if (kind != 1) p = (p * (kind == 2 ? xb : xa - 1)) / vol;
+            }
+            if constexpr (VM) {
+                if (L.vmx) {
+                    if (sp) L.vmx[l * WAVE + at] = x;
+                    sync_wave();
+                    // each lane its own program: a round, which runs them one after
+                    // the other, takes 120,000 cycles with 16 of them, an event
+                    // this way 24,000
+                    if (mine && kind == 4)
+                        p = vm_run<uint32_t, WAVE>(L.vcode, re->a, L.vk, L.vmx + at, vol, t,
+                                                   a.data_fn ? a.data_fn + (size_t)(up ? dv : sv) * a.n_df : nullptr);
+                }
+            }
+            if (re->mask && !((re->mask >> (up ? tds : tsv)) & 1ULL)) p = 0.0;
+            const double diff = p - r;
+            double rd = 0.0, rdd = 0.0;
+            for (unsigned h = dep; h; h &= h - 1) {
+                const int j = __builtin_ctz(h);
+                rd += rl_d(diff, j);
+                rdd += rl_d(diff, 32 + j);
+            }
+            if (mine) r = p;
+            sr += rd;
+            if (!react) srd += rdd;
+        }
+        if (!react) {
+            sd -= Dw;
+            sdd += Ddd;
+        }
+
+        // ---- the new firing times
+        unsigned long long pn = pos + (react ? 1 : 2);
+        double ntv = INFINITY, ntd = INFINITY;
+        int da = 0;
+        if (const double tot = sr + sd; __ballot(tot <= 0.0)) da--;
+        else ntv = expo(pn++) / tot + t;
+        if (!react) {
+            if (const double tot = srd + sdd; __ballot(tot <= 0.0)) {
+                if (__ballot(qtd != INFINITY)) da--;
+            } else {
+                ntd = expo(pn++) / tot + t;
+                if (__ballot(qtd == INFINITY)) da++;
+            }
+        }
+
+        // ---- store
+        const int at = up ? dv : sv;
+        if (side) {
+            if (sp && (react || l == which)) xx[(size_t)at * S + l] = x;
+            if (mine) rrate[(size_t)at * R + l] = r;
+            if (l == 0) {
+                srrate[at] = up ? srd : sr;
+                sdrate[at] = up ? sdd : sd;
+                qtime[at] = up ? ntd : ntv;
+            }
+        }
+        if (a.snap_tot && ((changed >> lane) & 1ULL)) atomicAdd(L.tot + l, (unsigned)d);
+        if (a.trace && lane == 0 && q.events_traced < a.trace_cap) {
+            ssasdpd_event ev;
+            ev.t = t; ev.voxel = sv; ev.kind = react ? 0 : 1; ev.which = which; ev.dest = react ? -1 : dv;
+            a.trace[q.events_traced] = ev;
+        }
+        pos = pn;
+        q.rxnCount++;
+        q.events_traced++;
+        if (react) q.reactions++;
+        else q.diffusions++;
+        q.active = (unsigned long long)((long long)q.active + da);
+
+        // ---- the queue
+        qtd = rl_d(qtd, 0);
+        ntv = rl_d(ntv, 0);
+        ntd = rl_d(ntd, 0);
+        remove(0);
+        if (!react) {
+            stale = dv;
+            if (qtd < INFINITY) {
+                if (!before(tau_t, tau_v, qtd, dv)) {
+                    const unsigned long long h = __ballot(lane < cnt && fv == dv);
+                    if (h) remove((int)__builtin_ctzll(h));
+                } else if (!before(far_t, far_v, qtd, dv)) {
+                    drop_near(dv);
+                }
+            }
+        }
+        if (ntv < INFINITY) insert(ntv, sv);
+        if (ntd < INFINITY) insert(ntd, dv);
+        return true;
+    }
 };
 
 }  // namespace
@@ -684,7 +937,8 @@ template <int MS, int MR, bool VM> struct Loop {
 // The event loop of one trajectory on one wavefront.  b: its index in a
 // batch that shares one argument block (strides bs_*), else 0.
 // VM: kind-4 reactions (custom propensities) through the expression VM.
-template <int MS, int MR, bool VM>
+// ALONE: where rounds keep too few events, they go one by one.
+template <int MS, int MR, bool VM, bool ALONE>
 __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
     extern __shared__ __align__(16) unsigned char smem[];
     QueueState *const qs_ = a.qs + b;
@@ -798,6 +1052,12 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
     lp.guess_empty = 1.0;
     const int widest = VM ? WAVE / 2 : WAVE;
     int width = widest;   // lanes a round tries: about twice what the last ones kept
+    // kept: 16 times what the last rounds kept, on average; below lone_at the
+    // next events go alone, 32 << lone of them, then a round to see.  lone_at: 16
+    // times a round's cost over an event's alone (2 at 2 species and reactions, 4
+    // at 8, 12 at 16: 10 x 10 voxels with 8 of each 54.8 ms in rounds, 54.5 so)
+    const int lone_at = VM ? 16 + 4 * R : MR <= 8 ? 24 + 11 * (S + R) / 4 : 6 * (S + R);
+    int kept = lone_at - 1, lone = 0;
     const bool textbook = a.textbook != 0;
     const double inf = INFINITY;
     int err = 0;
@@ -818,6 +1078,21 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
         const double end_time = t0 + a.dt;
         int stale = -1;                       // the last hop's destination
         unsigned long long guard = 0;
+        bool more = false;
+        do {
+        // events alone, as long as the front holds the next ones
+        if (ALONE && kept < lone_at) {
+            int left = 32 << lone;
+            for (; left > 0 && tt <= end_time && guard < a.max_events && lp.cnt > 0 &&
+                   !(lp.cnt < FRONT_LOW && lp.tau_t < inf); left--) {
+                const double first = rl_d(lp.ft, 0);
+                if (!(first <= q.U) || !lp.event_alone(q, stale)) break;
+                guard++;
+                tt = first;
+                sync_wave();
+            }
+        }
+        more = false;
         while (tt <= end_time) {
             if (guard >= a.max_events) { err = SSASDPD_ERR_CAPACITY; break; }
             // ---- selectReaction: the earliest voxel inside the window [L, U]
@@ -1247,6 +1522,11 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
             const bool done = act && lane < P;
             width = P == K ? min(2 * width, widest) : max(8, min(widest, (width + 3 * P + 8) / 2));
 
+            if (ALONE && (P < K || K == 1 || 16 * K >= lone_at)) {
+                kept += (16 * P - kept) / 8;
+                lone = kept < lone_at ? min(lone + 1, 5) : 0;
+            }
+
             // ---- store
             const unsigned long long m_done = __ballot(done), m_hop = __ballot(done && mv);
             if (done) {
@@ -1305,22 +1585,8 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 for (unsigned long long h = __ballot(inF); h; h &= h - 1)
                     gone |= __ballot(lane < lp.cnt && lp.fv == rl_i(dv, (int)__builtin_ctzll(h)));
                 for (unsigned long long h = __ballot(moved && !inF && !before(lp.far_t, lp.far_v, qtd, dv)); h;
-                     h &= h - 1) {
-                    // out of the near list: its last entry takes the place
-                    const int v = rl_i(dv, (int)__builtin_ctzll(h));
-                    for (int c0 = 0; c0 < lp.nc; c0 += WAVE) {
-                        const unsigned long long m = __ballot(c0 + lane < lp.nc && L.qv[c0 + lane] == v);
-                        if (!m) continue;
-                        lp.nc--;
-                        if (lane == 0) {
-                            const int k = c0 + (int)__builtin_ctzll(m);
-                            L.qt[k] = L.qt[lp.nc];
-                            L.qv[k] = L.qv[lp.nc];
-                        }
-                        sync_wave();
-                        break;
-                    }
-                }
+                     h &= h - 1)
+                    lp.drop_near(rl_i(dv, (int)__builtin_ctzll(h)));
                 const bool newS = done && ntv < inf, newD = done && mv && !self && ntd < inf;
                 const bool inS = newS && !before(lp.tau_t, lp.tau_v, ntv, sv);
                 const bool inD = newD && !before(lp.tau_t, lp.tau_v, ntd, dv);
@@ -1363,7 +1629,12 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
                 }
             }
             sync_wave();
+            if (ALONE && kept < lone_at) {
+                more = true;
+                break;
+            }
         }
+        } while (ALONE && more);
         if (err) { q.err_step = stp; break; }
     }
     if (!err)
@@ -1380,16 +1651,16 @@ __device__ __forceinline__ void ssa_run(const RdmeArgs &a, const size_t b) {
     if (lane == 0) *qs_ = q;
 }
 
-template <int MS, int MR, bool VM>
+template <int MS, int MR, bool VM, bool ALONE>
 __global__ void __launch_bounds__(WAVE * WAVES) k_ssa(RdmeArgs a) {
-    ssa_run<MS, MR, VM>(a, blockIdx.x);
+    ssa_run<MS, MR, VM, ALONE>(a, blockIdx.x);
 }
 
 // Ensembles of different models: workgroup g runs the trajectory described
 // by args[g] (its own domain, chemistry, queue and stream).
-template <int MS, int MR, bool VM>
+template <int MS, int MR, bool VM, bool ALONE>
 __global__ void __launch_bounds__(WAVE * WAVES) k_ssa_multi(const RdmeArgs *__restrict__ args) {
-    ssa_run<MS, MR, VM>(args[blockIdx.x], 0);
+    ssa_run<MS, MR, VM, ALONE>(args[blockIdx.x], 0);
 }
 
 // The per-lane tables are sized for 2, 4, 8 or 16 species and reactions (8 or
@@ -1417,21 +1688,46 @@ template <class K> static void allow_lds(K kernel, size_t lds) {
 // would only take the registers of other trajectories.
 static int threads_for(int n_traj) { return n_traj <= 256 ? WAVE * WAVES : WAVE; }
 
+// Whether a launch may take events alone: in domains of so few voxels that most
+// rounds keep fewer than they cost, and where that few voxels have a next event.
+// The lines (rounds / both ways, ms): up to 2 species and reactions, 16 voxels
+// 87.5 / 82.1, 25 voxels 71.5 / 74.2; up to 4, 25 voxels 60.2 / 52.0, 36 voxels
+// 57.1 / 57.8; up to 8, 64 voxels 76.1 / 60.8, 100 voxels 54.8 / 54.5, 144 voxels
+// 26.7 / 27.8; 16, 256 voxels 80.5 / 70.3, 400 voxels 100.8 / 100.6.  20,000
+// molecules in one of 3,600 voxels: 12.1 / 9.5.  Past them the kernel that only
+// knows rounds is 2% faster.  Custom propensities: 6 of them, 9 voxels 3.5 / 2.7,
+// 16 voxels 3.4 / 3.8; 8, 81 voxels 10.2 / 9.4, 169 voxels 19.7 / 17.0, 289 voxels
+// as in rounds; 16, 25 voxels 16.4 / 5.3, 289 voxels 99 / 68.
+bool nsm_alone(int n, int S, int R, bool vm, long long active) {
+    const int m = S > R ? S : R;
+    if (vm) return n <= (R <= 6 ? 9 : R <= 8 ? 150 : 300) || active <= 8;
+    return n <= (m <= 2 ? 20 : m <= 4 ? 32 : m <= 8 ? 100 : 256) || active <= 8;
+}
+
 void rdme_take_step(hipStream_t s, const RdmeArgs &a, int n_traj) {
     by_size(a.vm_ncode > 0, a.S > a.R ? a.S : a.R, [&](auto m, auto vm) {
         constexpr int M = decltype(m)::value;
         constexpr bool V = decltype(vm)::value;
-        allow_lds(k_ssa<M, M, V>, a.lds_bytes);
-        hipLaunchKernelGGL((k_ssa<M, M, V>), dim3(n_traj), dim3(threads_for(n_traj)), a.lds_bytes, s, a);
+        auto launch = [&](auto kernel) {
+            allow_lds(kernel, a.lds_bytes);
+            hipLaunchKernelGGL(kernel, dim3(n_traj), dim3(threads_for(n_traj)), a.lds_bytes, s, a);
+        };
+        if (a.alone) launch(k_ssa<M, M, V, true>);
+        else launch(k_ssa<M, M, V, false>);
     });
 }
 
-void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog) {
+void rdme_take_step_multi(hipStream_t s, const RdmeArgs *d_args, int n_models, int max_sr, size_t lds, bool any_prog,
+                          bool alone) {
     by_size(any_prog, max_sr, [&](auto m, auto vm) {
         constexpr int M = decltype(m)::value;
         constexpr bool V = decltype(vm)::value;
-        allow_lds(k_ssa_multi<M, M, V>, lds);
-        hipLaunchKernelGGL((k_ssa_multi<M, M, V>), dim3(n_models), dim3(threads_for(n_models)), lds, s, d_args);
+        auto launch = [&](auto kernel) {
+            allow_lds(kernel, lds);
+            hipLaunchKernelGGL(kernel, dim3(n_models), dim3(threads_for(n_models)), lds, s, d_args);
+        };
+        if (alone) launch(k_ssa_multi<M, M, V, true>);
+        else launch(k_ssa_multi<M, M, V, false>);
     });
 }
 
