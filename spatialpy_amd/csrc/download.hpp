@@ -12,8 +12,8 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -78,9 +78,12 @@ class Download {
         const int hw = (int)std::thread::hardware_concurrency();
         const int want = std::max(1, std::min(DOWNLOAD_THREADS, hw / 2));
         try {
+            team_.reserve(want);
             for (int k = 0; k < want; k++) team_.emplace_back([this] { work(); });
-        } catch (const std::system_error &) {
-            // as many as there are; with none the copies are plain ones
+        } catch (const std::exception &) {
+            // (std::system_error or std::bad_alloc: an exception that left here
+            // would destroy running threads.)  As many as there are; with none
+            // the copies are plain ones
         }
     }
     Download(const Download &) = delete;
