@@ -504,16 +504,18 @@ struct ssasdpd_engine {
         tree_nodes = (n + 64 * pl - 1) / (64 * pl);
         dfree(tmin);
         tmin = dalloc<double>(tree_nodes);
-        if (admitted_lds(p) > 65536)
+        if (!lds_ok(p))
             throw HipError("event-loop constants exceed 64 KiB of LDS", hipErrorUnknown, __FILE__, __LINE__);
-        lds_bytes = nsm_lds_bytes(tree_nodes, S, R, T, n_code, n_consts);
+        lds_bytes = lds_at(p);
     }
-    // ssa_lds_bytes at node width p, over a tree of the nodes and of the
-    // levels above them, 64 to one
-    size_t admitted_lds(int p) const {
+    // The event loop's LDS at node width p.
+    size_t lds_at(int p) const { return nsm_lds_bytes((n + 64 * p - 1) / (64 * p), S, R, T, n_code, n_consts); }
+    // Whether a model's tables are accepted at node width p (ssa_lds_bytes, with
+    // a tree of the nodes and of the levels above them, 64 to one), and fit.
+    bool lds_ok(int p) const {
         int n1 = (n + 64 * p - 1) / (64 * p), nodes = n1;
         while (n1 > 1) { n1 = (n1 + TREE_FAN - 1) / TREE_FAN; nodes += n1; }
-        return ssa_lds_bytes(nodes, S, R, T, nnzN_, nnzG_, n_code, n_consts);
+        return ssa_lds_bytes(nodes, S, R, T, nnzN_, nnzG_, n_code, n_consts) <= 65536 && lds_at(p) <= LDS_MAX;
     }
     // Change the node width of a built queue: the bounds are formed again from
     // the firing times, so the event sequence is unchanged.
@@ -703,7 +705,7 @@ struct ssasdpd_engine {
             layout_tree(p0);
             vol = dalloc<double>(n);
             qs = dalloc<QueueState>(1);
-qwork = dalloc<char>(q_work_bytes(n));
+            qwork = dalloc<char>(q_work_bytes(n));
         }
         if (Sc > 0 && Rc > 0 && d->N_dense) {
             Ndense = dalloc<int>((size_t)Sc * Rc);
@@ -1538,7 +1540,7 @@ struct ssasdpd_ensemble {
         for (auto *e : eng)
             if (!ssasdpd_engine::pl_valid(p, e->n)) return false;
         for (auto *e : eng)
-            if (e->admitted_lds(p) > 65536) return false;
+            if (!e->lds_ok(p)) return false;
         return true;
     }
     void set_pl(int p) {

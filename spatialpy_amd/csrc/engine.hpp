@@ -354,6 +354,10 @@ void vm_eval_batch(hipStream_t s, const uint32_t *code, int start, const double 
 // Row permutation of an [n][cols] array of esz-byte elements (4 or 8):
 // gather dst[p] = src[map[p]], or scatter dst[map[p]] = src[p] (sdpd.hip).
 void permute_rows(hipStream_t s, int n, int cols, int esz, const int *map, const void *src, void *dst, bool scatter);
+// The event loop's LDS, of a CU's LDS_MAX; and the size, at most 64 KiB, by
+// which models have been accepted since the event queue was a tree in LDS with
+// (time, voxel) at every node.  The first is at most some 36 KiB larger.
+constexpr size_t LDS_MAX = 160 << 10;
 size_t nsm_lds_bytes(int nodes, int S, int R, int T, int n_code, int n_consts);
 size_t ssa_lds_bytes(int tree_nodes, int S, int R, int T, int nnzN, int nnzG, int n_code = 0, int n_consts = 0);
 

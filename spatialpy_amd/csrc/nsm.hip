@@ -7,7 +7,7 @@
 // instructions, 3-4 us, with one lane's worth of work in a 64-lane wavefront.
 // But consecutive events rarely touch each other: of the next 64 events in
 // firing order, those before the first one that shares a voxel with an
-// earlier one (30 on average on a 2D dam break with 1,000 molecules, 60 on a
+// earlier one (26 on average on a 2D dam break with 1,000 molecules, 51 on a
 // 64,000-voxel lattice, 6 on 121 voxels) can be carried out side by side.
 // So each round
 //   1. takes the earliest voxels of the queue, one per lane, in firing order;

@@ -1,25 +1,22 @@
-// GPU-resident NSM (next-subvolume method) for the sSSA part.
+// Rates and event queue of the NSM (next-subvolume method), the sSSA part; the
+// event loop is in nsm.hip.
 //
-//   rdme_rates        nsm_core__initialize_rxn_propensities and
-//                     nsm_core__initialize_diff_propensities
-//                     (ENG/src/simulate_rdme.cpp:113-152)
-//   rdme_queue_build  nsm_core__initialize_heap + NRMConstant_v5::build
-//                     (simulate_rdme.cpp:155-195, NRMConstant_v5.cpp:27-85)
-//   rdme_take_step    nsm_core__take_step (simulate_rdme.cpp:211-472)
+//   rdme_queue_build  nsm_core__initialize_rxn_propensities,
+//                     nsm_core__initialize_diff_propensities and
+//                     nsm_core__initialize_heap + NRMConstant_v5::build
+//                     (ENG/src/simulate_rdme.cpp:113-195,
+//                     NRMConstant_v5.cpp:27-85), for all trajectories of a
+//                     batch in three launches or four
+//   rdme_diag         the diffusion sums over the neighbour rows
+//   tree_rebuild      the queue's node bounds after a change of their width
 //
-// The event queue is an indexed min-tree over the voxels' firing times:
-// F0 = 64*PL voxels under each level-1 node, 64 nodes under each node above
-// (one wavefront reduces one node).  The levels above the voxels live in LDS
-// while the event loop runs.  The reference's time-binned hash
-// table always yields the global minimum among firing times inside its
-// current window [L, U] and rebuilds the window when that set is empty
-// (NRMConstant_v5.cpp:156-281); the window scalars are kept here with the
-// same update rules, so the min-tree returns the same event sequence (up to
-// exactly equal firing times, which the table breaks by bin order).
-//
-// One 64-lane workgroup runs one trajectory's event loop; every lane
-// executes the scalar logic (uniform control flow, broadcast loads), lanes
-// split the min-tree node reductions and the neighbour-row loads.
+// The queue is the voxels' firing times and the minimum of every node of
+// 64*pl voxels.  The reference's time-binned hash table always yields the
+// global minimum among the firing times inside its current window [L, U] and
+// rebuilds the window when that set is empty (NRMConstant_v5.cpp:156-281); the
+// window's scalars are kept with the same update rules (window.hpp), so the
+// event sequence is the same (up to exactly equal firing times, which the
+// table breaks by bin order).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -372,8 +369,9 @@ void vm_eval_batch(hipStream_t s, const uint32_t *code, int start, const double 
                        n_x, n_df, m, xd, xu, vol, t, df, out);
 }
 
-// What the library accepts as an event-loop model: the tables of its chemistry
-// and programs beside a tree of tree_nodes (time, voxel) pairs, up to 64 KiB.
+// What the library accepts as an event-loop model, up to 64 KiB: the tables of
+// its chemistry and programs beside tree_nodes (time, voxel) pairs, as a tree of
+// them once stood in LDS.  (What the loop uses now is nsm_lds_bytes.)
 size_t ssa_lds_bytes(int tree_nodes, int S, int R, int T, int nnzN, int nnzG, int n_code, int n_consts) {
     auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
     size_t off = 0;
