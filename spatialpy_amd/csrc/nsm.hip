@@ -53,9 +53,9 @@
 // cylinder, 860 events a step, 2.8 -> 0.45 us; 121 voxels 3.5 -> 1.5 us;
 // custom propensities on 144 voxels 30 -> 5.2 us; 4 voxels 3.6 -> 5.5 us in
 // rounds, 3.0 us one by one (16 voxels with 16 species and 16 reactions 4.3 ->
-// 16.4 and 3.7 us).  A round takes 20,000 to
-// 50,000 cycles, most of them latencies (two round trips, LDS, dependent
-// FP64 operations) of a single wavefront.
+// 16.4 and 3.7 us).  A round takes 20,000 to 50,000 cycles, most of them
+// latencies (two round trips, LDS, dependent FP64 operations) of a single
+// wavefront.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -1695,12 +1695,13 @@ static int threads_for(int n_traj) { return n_traj <= 256 ? WAVE * WAVES : WAVE;
 // 57.1 / 57.8; up to 8, 64 voxels 76.1 / 60.8, 100 voxels 54.8 / 54.5, 144 voxels
 // 26.7 / 27.8; 16, 256 voxels 80.5 / 70.3, 400 voxels 100.8 / 100.6.  20,000
 // molecules in one of 3,600 voxels: 12.1 / 9.5.  Past them the kernel that only
-// knows rounds is 2% faster.  Custom propensities: 6 of them, 9 voxels 3.5 / 2.7,
-// 16 voxels 3.4 / 3.8; 8, 81 voxels 10.2 / 9.4, 169 voxels 19.7 / 17.0, 289 voxels
-// as in rounds; 16, 25 voxels 16.4 / 5.3, 289 voxels 99 / 68.
+// knows rounds is 2% faster.  Custom propensities: 6 of them, 4 voxels 3.5 / 2.7,
+// 9 voxels 3.6 / 3.1 or, with exp and pow in them, 3.4 / 3.8; 8, 64 voxels 10.2 /
+// 9.4, 144 voxels 19.7 / 17.0; 16, 16 voxels 16.4 / 5.3, 256 voxels 99 / 68, 576
+// voxels 171 / 168.
 bool nsm_alone(int n, int S, int R, bool vm, long long active) {
     const int m = S > R ? S : R;
-    if (vm) return n <= (R <= 6 ? 9 : R <= 8 ? 150 : 300) || active <= 8;
+    if (vm) return n <= (R <= 6 ? 4 : R <= 8 ? 150 : 300) || active <= 8;
     return n <= (m <= 2 ? 20 : m <= 4 ? 32 : m <= 8 ? 100 : 256) || active <= 8;
 }
 
