@@ -66,21 +66,7 @@ __device__ __forceinline__ void store_rec_to(const SdpdArgs &a, int i, double2 *
 }
 __device__ __forceinline__ void store_rec(const SdpdArgs &a, int i) { store_rec_to(a, i, (double2 *)(a.rec + i)); }
 
-// Neighbour j's record: x, v, vt, nu, rho, mass (six 16-byte loads of one
-// 128-byte line).
-__device__ __forceinline__ void load_rec(const PRec *r, double x[3], double v[3], double vt[3], double &nu,
-                                         double &rho, double &mass) {
-    const double2 *p = (const double2 *)r;
-    const double2 a0 = p[0], a1 = p[1], a2 = p[2], a3 = p[3], a4 = p[4], a5 = p[5];
-    x[0] = a0.x; x[1] = a0.y; x[2] = a1.x;
-    v[0] = a1.y; v[1] = a2.x; v[2] = a2.y;
-    vt[0] = a3.x; vt[1] = a3.y; vt[2] = a4.x;
-    nu = a4.y; rho = a5.x; mass = a5.y;
-}
-
 __device__ __forceinline__ double2 load_rho_mass(const PRec *r) { return *(const double2 *)&r->rho; }
-// P_j / rho_j^2 and m_j / rho_j of the record (see store_rec_to)
-__device__ __forceinline__ double2 load_rec_pm(const PRec *r) { return ((const double2 *)r)[7]; }
 
 __global__ void k_pack(SdpdArgs a) {
     const int chunk = xcd_chunk((a.n + 255) / 256);

@@ -53,7 +53,7 @@ class Ensemble:
         _abi.check(self.lib, self.lib.ssasdpd_ensemble_set_tree_width(self.h, int(pl)), "set_tree_width")
 
     def autotune(self, seeds, probe_steps=2):
-        """Time probe_steps steps at each event-tree width and keep the
+        """Time probe_steps steps at each event-queue width and keep the
         fastest.  Returns (chosen width, {width: GPU ms})."""
         seeds = np.ascontiguousarray(np.asarray(seeds, dtype=np.uint64))
         ms = np.zeros(4)
